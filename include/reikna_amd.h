@@ -268,6 +268,12 @@ int rk_fft_plan_num_passes(const rk_fft_plan* plan, int* n);
    before the next chunk starts (of *n_outer); 0 when the plan is not chunked. */
 int rk_fft_plan_chunking(const rk_fft_plan* plan, int64_t* chunk_outer, int64_t* n_outer);
 int rk_fft_plan_pass_info(const rk_fft_plan* plan, int pass, rk_fft_pass_info* info);
+/* Instances per tile of the kernel that computes two adjacent instances per
+   thread, when the pass runs it (0: it does not).  rk_fft_pass_info's C,
+   threads, grid and lds_bytes are those of the one-instance-per-thread tile:
+   the geometry of a kernel set with rk_fft_plan_set_pass_kernel, which then
+   runs instead. */
+int rk_fft_plan_pass_pair(const rk_fft_plan* plan, int pass, int* instances);
 
 /* Replace the kernel of one pass with a run-time compiled one whose
    parameter list is the same pass-argument struct (fused transformations). */

@@ -272,6 +272,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "rk_fft_plan_num_passes": (_I, [_P, ctypes.POINTER(_I)]),
     "rk_fft_plan_chunking": (_I, [_P, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)]),
     "rk_fft_plan_pass_info": (_I, [_P, _I, ctypes.POINTER(FftPassInfo)]),
+    "rk_fft_plan_pass_pair": (_I, [_P, _I, ctypes.POINTER(_I)]),
     "rk_fft_plan_set_pass_kernel": (_I, [_P, _I, _P]),
     "rk_fft_plan_set_timing": (_I, [_P, _I]),
     "rk_fft_plan_pass_time_ms": (_I, [_P, _I, ctypes.POINTER(ctypes.c_float)]),

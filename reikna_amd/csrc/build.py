@@ -115,6 +115,13 @@ def tile_c_col(length: int) -> int:
     return c
 
 
+def pair_tile_widths(length: int) -> list[int]:
+    """Instances per tile of a pair kernel: 16 .. 64 with at most 256 threads
+    (16 always), as rk_fft_plan.cpp pair_tile picks them."""
+    t = threads_per_instance(length)
+    return [c for c in (16, 32, 64) if c == 16 or c // 2 * t <= 256]
+
+
 def catalog_lengths() -> list[int]:
     ls = set()
     ls.update(2**k for k in range(1, 15))
@@ -140,6 +147,8 @@ VAR_MODE_FF = 1 << 10                # load/store modes FLAT/FLAT compiled in (R
 VAR_NT_LOAD = 1 << 11                # nontemporal loads only (RK_VAR_NT_LOAD)
 VAR_NT_STORE = 1 << 12               # nontemporal stores only (RK_VAR_NT_STORE)
 VAR_OCC = 1 << 16                    # launch bounds for the LDS-allowed residency (RK_VAR_OCC)
+PAIR_MIN = 512                       # shortest pass with two instances per thread (rk_fft_plan.cpp pair_tile)
+VAR_PAIR = 1 << 18                   # two adjacent instances per thread (RK_VAR_PAIR)
 FACTOR_MAX = 1024                    # longest pass of a complex64 multi-pass chain (rk_fft_plan.cpp factor_max)
 
 
@@ -206,6 +215,14 @@ def catalog_entries() -> list[tuple[int, int, int]]:
         if (length <= 1024 and c * threads_per_instance(length) == 1024 and base in (VAR_PLAIN, VAR_TWIDDLE)
                 and v & (VAR_MODE_DD | VAR_MODE_DF)):
             ents.add((length, c, v | VAR_OCC))
+    # the power-of-two column passes with two instances per thread
+    # (rk_fft_plan.cpp pair_tile), for every tile width the planner may pick
+    for length, c, v in list(ents):
+        base = v & ~(nt | VAR_MODE_DD | VAR_MODE_DF)
+        if (length & (length - 1) == 0 and PAIR_MIN <= length <= FACTOR_MAX and c == tile_c_col(length)
+                and base in (VAR_PLAIN, VAR_TWIDDLE) and v & (VAR_MODE_DD | VAR_MODE_DF)):
+            for cp in pair_tile_widths(length):
+                ents.add((length, cp, v | VAR_PAIR))
     # single-pass row tiles of such lengths (one thread per R0 elements of an
     # instance, at least 32 of them: shorter rows are streamed flat): the
     # 1000-point tile holds 80 VGPRs with every mode and 62 with DIRECT/DIRECT
@@ -317,15 +334,15 @@ def generate_catalog(out_dir: Path) -> list[Path]:
             '#include "rk_internal.hpp"',
             f"namespace rk_catalog_{k} {{",
             "template <int L, int C, int V>",
-            "__global__ void __launch_bounds__((rkfft::pass_threads<L, C>()), (rkfft::pass_min_waves<L, C, V>()))",
+            "__global__ void __launch_bounds__((rkfft::variant_threads<L, C, V>()), (rkfft::pass_min_waves<L, C, V>()))",
             "rk_fft_pass(rk_pass_args a) {",
             "    rkfft::fft_pass_entry<L, C, V>(a);",
             "}",
             "static const rk::KernelEntry entries[] = {",
         ]
         for length, c, v in sorted(part):
-            threads = c * threads_per_instance(length)
-            lds = tile_lds_bytes(length, c)
+            threads = c // (2 if v & VAR_PAIR else 1) * threads_per_instance(length)
+            lds = tile_lds_bytes(length, c // (2 if v & VAR_PAIR else 1))
             lines.append(
                 f"    {{{length}, {c}, {v}, {threads}, {lds}, "
                 f"(const void*)&rk_fft_pass<{length}, {c}, {v}>}},"

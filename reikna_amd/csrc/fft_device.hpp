@@ -44,18 +44,42 @@ namespace rkfft {
 // complex arithmetic (x = re, y = im) on complex64 (float2) and complex128
 // (double2) values; a pass's element type is its IO policy's value_type
 // ------------------------------------------------------------------------
+template <class F> using rk_v2 = F __attribute__((ext_vector_type(2)));
+
+// The values of two adjacent instances at one position, part by part: a pass
+// whose value type is cpair2 computes two instances per thread with the same
+// code (elementwise arithmetic; PairIO below).
+struct cpair2 {
+    rk_v2<float> x, y;
+};
+
 template <class X> struct RealOf;
 template <> struct RealOf<float2> { typedef float type; };
 template <> struct RealOf<double2> { typedef double type; };
+template <> struct RealOf<cpair2> { typedef rk_v2<float> type; };
 template <class X> using real_t = typename RealOf<X>::type;
+
+// Instances per thread of a value type, and its single complex value (the
+// element type of its tables).
+template <class X> struct ScalarOf { typedef X type; };
+template <> struct ScalarOf<cpair2> { typedef float2 type; };
+template <class X> using scalar_t = typename ScalarOf<X>::type;
+template <class X> RK_HD constexpr int pair_width() { return (int)(sizeof(X) / sizeof(scalar_t<X>)); }
 
 template <class X> RK_HD X cx(real_t<X> re, real_t<X> im);
 template <> RK_HD float2 cx<float2>(float re, float im) { return make_float2(re, im); }
 template <> RK_HD double2 cx<double2>(double re, double im) { return make_double2(re, im); }
+template <> RK_HD cpair2 cx<cpair2>(rk_v2<float> re, rk_v2<float> im) {
+    cpair2 r;
+    r.x = re;
+    r.y = im;
+    return r;
+}
 
 template <class X> RK_HD X c_add(X a, X b) { return cx<X>(a.x + b.x, a.y + b.y); }
 template <class X> RK_HD X c_sub(X a, X b) { return cx<X>(a.x - b.x, a.y - b.y); }
-template <class X> RK_HD X c_mul(X a, X b) { return cx<X>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// b: a value of the same type, or one complex factor for both of a cpair2's
+template <class X, class W> RK_HD X c_mul(X a, W b) { return cx<X>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 template <class X> RK_HD X c_conj(X a) { return cx<X>(a.x, -a.y); }
 template <class X> RK_HD X c_mul_mi(X a) { return cx<X>(a.y, -a.x); }   // a * (-i)
 template <class X> RK_HD X c_scale(X a, real_t<X> s) { return cx<X>(a.x * s, a.y * s); }
@@ -328,6 +352,18 @@ RK_HD constexpr int lds_pitch_for(int L, int C, int T, bool force_split = false,
     return p;
 }
 
+// Row pitch (in 64-bit slots) and LDS bytes of a pair tile of C instances:
+// C/2 rows of 64-bit values, the pitch rule of 64-bit accesses above.
+RK_HD constexpr int lds_pitch_pair(int L, int C, int T) {
+    const int CP = C / 2;
+    const bool pow2 = CP > 0 && (CP & (CP - 1)) == 0;
+    if (!pow2 || CP < 2 || T < 16 || CP > 16) return lds_pitch_base(L);
+    int p = lds_pad(L - 1) + 1;
+    while (p % 32 != 32 / CP) ++p;
+    return p;
+}
+RK_HD constexpr int pair_lds_bytes(int L, int C, int T) { return (C / 2) * lds_pitch_pair(L, C, T) * 8; }
+
 // ------------------------------------------------------------------------
 // per-instance coordinates
 // ------------------------------------------------------------------------
@@ -369,6 +405,10 @@ __device__ __forceinline__ Inst decompose(const rk_pass_args& a, rk_u64 inst) {
     return r;
 }
 
+// Axis position of a pair's second instance minus its first's: pairs are
+// adjacent along the innermost of the dims I, NS, H that is longer than one.
+__device__ __forceinline__ rk_u64 pair_step(const rk_pass_args& a) { return a.dim_I > 1 ? 0 : 1; }
+
 // W_N^e for 0 <= e < N from two FP64 tables; the product is formed in FP64
 // and rounded once to the element's real type.
 __device__ __forceinline__ double2 d_mul(double2 a, double2 b) {
@@ -409,14 +449,47 @@ __device__ __forceinline__ void apply_pass_twiddles(const rk_pass_args& a, rk_u6
     for (int r = 0; r < NV; ++r) x[r] = c_mul(x[r], tw.template next<X>());
 }
 
+// Two instances per thread: one walk per instance (equal when the pair
+// differs in its inner batch index only).
+template <int NV>
+__device__ __forceinline__ void apply_pass_twiddles(const rk_pass_args& a, rk_u64 l, int p0, int dp, cpair2* x) {
+    TwiddleWalk tw0, tw1;
+    tw0.init(a, l, (rk_u64)p0, (rk_u64)dp);
+    tw1.init(a, l + pair_step(a), (rk_u64)p0, (rk_u64)dp);
+#pragma unroll
+    for (int r = 0; r < NV; ++r) {
+        const float2 w0 = tw0.template next<float2>(), w1 = tw1.template next<float2>();
+        cpair2 w;
+        w.x = rk_v2<float>{w0.x, w1.x};
+        w.y = rk_v2<float>{w0.y, w1.y};
+        x[r] = c_mul(x[r], w);
+    }
+}
+
 // The table pointers of the pass arguments, as the element type X of a pass
 // (complex64 or complex128 tables; the host builds the ones its plan needs).
-template <class X> __device__ __forceinline__ const X* table(const float2* p) { return reinterpret_cast<const X*>(p); }
+template <class X> __device__ __forceinline__ const scalar_t<X>* table(const float2* p) {
+    return reinterpret_cast<const scalar_t<X>*>(p);
+}
+
+// Entry k of a table for a value of type X: of a pair, the entries k and k2
+// of its two instances.
+template <class X> __device__ __forceinline__ X table_at(const float2* p, rk_u64 k, rk_u64 k2) {
+    if constexpr (pair_width<X>() == 2) {
+        const float2 w0 = p[k], w1 = p[k2];
+        cpair2 w;
+        w.x = rk_v2<float>{w0.x, w1.x};
+        w.y = rk_v2<float>{w0.y, w1.y};
+        return w;
+    } else {
+        return table<X>(p)[k];
+    }
+}
 
 // The output scale (1/N on the last pass of an inverse transform) in the
 // element's real type: complex128 passes take the FP64 value.
 template <class X> __device__ __forceinline__ real_t<X> out_scale_of(const rk_pass_args& a) {
-    if constexpr (sizeof(real_t<X>) == 8) return a.out_scale64;
+    if constexpr (sizeof(real_t<scalar_t<X>>) == 8) return a.out_scale64;
     else return a.out_scale;
 }
 
@@ -441,7 +514,6 @@ template <class X> __device__ __forceinline__ real_t<X> out_scale_of(const rk_pa
 // intermediate stays in that cache between passes streams only its first
 // pass's loads and its last pass's stores.  X is the element type
 // (complex64 float2, complex128 double2); every IO policy names it value_type.
-template <class F> using rk_v2 = F __attribute__((ext_vector_type(2)));
 template <bool NTL, bool NTS = NTL, class X = float2> struct GlobalIO {
     using value_type = X;
     static constexpr bool kBranchFree = true;
@@ -470,6 +542,42 @@ template <bool NTL, bool NTS = NTL, class X = float2> struct GlobalIO {
 };
 using PlainIO = GlobalIO<false>;
 using StreamIO = GlobalIO<true>;
+
+// Two adjacent instances per thread (complex64, column tiles): their elements
+// at one position are neighbours in memory, so a load or store moves 16 bytes
+// per lane, half as many vector-memory instructions per element.  The element
+// address need not be 16-byte aligned (an instance pair starts at any even
+// element of the caller's view).
+typedef float rk_v4u __attribute__((ext_vector_type(4), aligned(8)));
+template <bool NTL, bool NTS = NTL> struct PairIO {
+    using value_type = cpair2;
+    static constexpr bool kBranchFree = true;
+    __device__ __forceinline__ cpair2 load(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*m*/, rk_u64 /*i*/,
+                                           rk_i64 addr) const {
+        const rk_v4u* p = reinterpret_cast<const rk_v4u*>(a.in + addr);
+        rk_v4u v;
+        if constexpr (NTL) v = __builtin_nontemporal_load(p);
+        else v = *p;
+        return cx<cpair2>(rk_v2<float>{v.x, v.z}, rk_v2<float>{v.y, v.w});
+    }
+    // one instance's element (padded sides, where a pair may straddle the edge)
+    __device__ __forceinline__ float2 load_one(const rk_pass_args& a, rk_i64 addr) const { return a.in[addr]; }
+    // two consecutive complex values at addr
+    __device__ __forceinline__ void store_run(const rk_pass_args& a, rk_i64 addr, float x0, float y0, float x1,
+                                              float y1) const {
+        rk_v4u* p = reinterpret_cast<rk_v4u*>(a.out + addr);
+        const rk_v4u v = {x0, y0, x1, y1};
+        if constexpr (NTS) __builtin_nontemporal_store(v, p);
+        else *p = v;
+    }
+    __device__ __forceinline__ void store(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*k*/, rk_u64 /*i*/, rk_i64 addr,
+                                          cpair2 v) const {
+        store_run(a, addr, v.x.x, v.y.x, v.x.y, v.y.y);
+    }
+    __device__ __forceinline__ void store_one(const rk_pass_args& a, rk_i64 addr, float x, float y) const {
+        a.out[addr] = make_float2(x, y);
+    }
+};
 
 // Plain strided IO whose loads and stores are coherent across the whole
 // device (relaxed agent-scope atomics: they bypass the caches that are not
@@ -539,6 +647,9 @@ struct CoherentIO {
 // Bit of a kernel's variant number: complex128 elements (FP64 butterflies,
 // twiddles and tables); such kernels come from the run-time compiler only.
 #define RK_VAR_F64 131072
+// Bit of a kernel's variant number: two adjacent instances per thread (PairIO;
+// DIRECT/DIRECT or DIRECT/FLAT compiled in, complex64).
+#define RK_VAR_PAIR 262144
 // MODES template argument of fft_pass_tile: 0 reads the modes from the pass
 // arguments, RK_MODES(load, store) compiles them in.
 #define RK_MODES(load, store) (16 | (int)(load) | ((int)(store) << 2))
@@ -594,7 +705,17 @@ __device__ __forceinline__ typename IO::value_type load_at(const rk_pass_args& a
     const rk_u64 m = w.m0 + (rk_u64)c * w.mstep;
     const rk_i64 addr = w.a0 + (rk_i64)c * w.astep;
     const X zero = cx<X>((real_t<X>)0, (real_t<X>)0);
-    if constexpr (pad_in<V>()) {
+    if constexpr (pad_in<V>() && pair_width<X>() == 2) {
+        // the pair may straddle the edge of the data: one load per instance,
+        // each at its own address or its instance's first position
+        const rk_u64 st = pair_step(a);
+        const rk_i64 next = ic.in_base + (rk_i64)(m + st) * a.in_sa + (st ? 0 : a.in_si);
+        const bool ok0 = ic.valid && m < a.n_valid_in, ok1 = ic.valid && m + st < a.n_valid_in;
+        const rk_u64 spare_m = ic.jpass < a.n_valid_in ? ic.jpass : 0;
+        const rk_i64 spare = ic.in_base + (rk_i64)spare_m * a.in_sa;
+        const float2 v0 = io.load_one(a, ok0 ? addr : spare), v1 = io.load_one(a, ok1 ? next : spare);
+        return cx<X>(rk_v2<float>{ok0 ? v0.x : 0.0f, ok1 ? v1.x : 0.0f}, rk_v2<float>{ok0 ? v0.y : 0.0f, ok1 ? v1.y : 0.0f});
+    } else if constexpr (pad_in<V>()) {
         const bool ok = ic.valid && m < a.n_valid_in;
         if constexpr (IO::kBranchFree) {
             // a lane with nothing to load reads its instance's first position
@@ -632,7 +753,8 @@ __device__ __forceinline__ void pre_ops(const rk_pass_args& a, const Inst& ic, c
         for (int i = 0; i < NV; ++i) {
             const rk_u64 m = w.m0 + (rk_u64)cpos(i) * w.mstep;
             const bool ok = ic.valid && m < a.n_valid_in;
-            x[i] = c_mul(x[i], table<X>(a.chirp)[ok ? m : 0]);
+            const rk_u64 m2 = m + pair_step(a);
+            x[i] = c_mul(x[i], table_at<X>(a.chirp, ok ? m : 0, m2 < a.n_valid_in ? m2 : 0));
         }
     }
 }
@@ -645,10 +767,10 @@ template <class X> __device__ __forceinline__ X adjust_out(const rk_pass_args& a
 }
 
 template <int V, class X>
-__device__ __forceinline__ X post_op(const rk_pass_args& a, rk_u64 kabs, X y, bool adjust) {
+__device__ __forceinline__ X post_op(const rk_pass_args& a, rk_u64 kabs, rk_u64 kabs2, X y, bool adjust) {
     constexpr int POST = Variant<V>::POST;
-    if constexpr (POST == RK_VAR_POST_KMUL_CONJ) y = c_conj(c_mul(y, table<X>(a.bspec)[kabs]));
-    if constexpr (POST == RK_VAR_POST_CONJ_CHIRP) y = c_mul(c_conj(y), table<X>(a.chirp)[kabs]);
+    if constexpr (POST == RK_VAR_POST_KMUL_CONJ) y = c_conj(c_mul(y, table_at<X>(a.bspec, kabs, kabs2)));
+    if constexpr (POST == RK_VAR_POST_CONJ_CHIRP) y = c_mul(c_conj(y), table_at<X>(a.chirp, kabs, kabs2));
     if (adjust) y = adjust_out(a, y);
     return y;
 }
@@ -658,10 +780,21 @@ __device__ __forceinline__ X post_op(const rk_pass_args& a, rk_u64 kabs, X y, bo
 template <int V, class IO>
 __device__ __forceinline__ void store_at(const rk_pass_args& a, const IO& io, const Inst& ic, const Walk& w, int c,
                                          typename IO::value_type y, bool adjust) {
+    using X = typename IO::value_type;
     const rk_u64 kabs = w.m0 + (rk_u64)c * w.mstep;
     if constexpr (pad_out<V>())
         if (kabs >= a.n_valid_out) return;
-    io.store(a, ic.o, kabs, ic.i, w.a0 + (rk_i64)c * w.astep, post_op<V>(a, kabs, y, adjust));
+    // a DIRECT store's pair is adjacent along I, or along NS (position + 1)
+    const rk_u64 k2 = kabs + (pair_width<X>() == 2 ? pair_step(a) : 0);
+    const rk_i64 addr = w.a0 + (rk_i64)c * w.astep;
+    if constexpr (pad_out<V>() && pair_width<X>() == 2) {
+        const bool two = k2 < a.n_valid_out;
+        y = post_op<V>(a, kabs, two ? k2 : kabs, y, adjust);
+        if (two) io.store(a, ic.o, kabs, ic.i, addr, y);
+        else io.store_one(a, addr, y.x.x, y.y.x);
+    } else {
+        io.store(a, ic.o, kabs, ic.i, addr, post_op<V>(a, kabs, k2, y, adjust));
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -824,10 +957,26 @@ RK_HD constexpr int flat_lds(int tid, int it) {
 
 // Padded LDS position of element it of a thread at position ps < T of an
 // instance on a staged COLUMN / ROW side: ps + it*T.
+// The same for a pair tile, whose threads take two consecutive positions at a
+// time: value 2*it + b is position e % L + b of pair e / L, e = 2*(tid + it*NT)
+// (L even, so both positions are on one side of every padding slot).
+template <int L, int NT, int LP>
+RK_HD constexpr int flat_pair_lds(int tid, int it, int b) {
+    if constexpr ((2 * NT) % L == 0) {
+        return ((2 * tid) / L) * LP + lds_pad((2 * tid) % L) + it * ((2 * NT) / L) * LP + b;
+    } else if constexpr (L % (2 * NT) == 0) {
+        return ((it * 2 * NT) / L) * LP + lds_pad_add<(2 * NT < 16 ? 2 * NT : 16)>(2 * tid, (it * 2 * NT) % L) + b;
+    } else {
+        const int e = 2 * (tid + it * NT);
+        const int ce = e / L;
+        return ce * LP + lds_pad(e - ce * L) + b;
+    }
+}
+
 template <int T> RK_HD constexpr int col_lds(int ps, int it) { return lds_pad_add<(T < 16 ? T : 16)>(ps, it * T); }
 
 template <int L, int S, bool SPLIT, int VM, bool WAVE = false, class X>
-__device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const X* twl) {
+__device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const scalar_t<X>* twl) {
     using P = Plan<L>;
     constexpr int R = P::radix(S);
     constexpr int NS = P::ns(S);
@@ -891,6 +1040,21 @@ template <int L, int C, bool HALF = false, int ES = 8> __host__ __device__ const
     return C * tile_pitch<L, C, HALF, ES>() * (tile_split<L, C, HALF, ES>() ? ES / 2 : ES);
 }
 
+// The same of a pass's value type.  A pair tile of C instances has C/2 pairs
+// and exchanges real parts, then imaginary parts, of both instances of a pair
+// as 64-bit values: its LDS is that of a whole (unsplit) tile of C/2 instances.
+template <int L, int C, bool HALF, class X> __host__ __device__ constexpr bool tile_split_x() {
+    return pair_width<X>() == 2 || tile_split<L, C, HALF, (int)sizeof(scalar_t<X>)>();
+}
+template <int L, int C, bool HALF, class X> __host__ __device__ constexpr int tile_pitch_x() {
+    if (pair_width<X>() == 2) return lds_pitch_pair(L, C, Plan<L>::T);
+    return tile_pitch<L, C, HALF, (int)sizeof(scalar_t<X>)>();
+}
+template <int L, int C, bool HALF, class X> __host__ __device__ constexpr int tile_lds_bytes_x() {
+    if (pair_width<X>() == 2) return pair_lds_bytes(L, C, Plan<L>::T);
+    return tile_lds_bytes<L, C, HALF, (int)sizeof(scalar_t<X>)>();
+}
+
 // One tile (instances tile*C ... tile*C + C - 1) computed by threads
 // tid = 0 ... C*T - 1 with `lds` of at least tile_lds_bytes<L, C, HALF, ES>()
 // bytes (ES = sizeof the IO policy's element type).
@@ -904,42 +1068,46 @@ template <int L, int C, int V, class IO, int MODES = 0, bool WAVE = false, bool 
           bool TWLDS = false>
 __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& io, typename IO::value_type* lds,
                                               rk_u64 tile, int tid, const typename IO::value_type* pre = nullptr,
-                                              const typename IO::value_type* twl_lds = nullptr) {
+                                              const scalar_t<typename IO::value_type>* twl_lds = nullptr) {
     using X = typename IO::value_type;
     using F = real_t<X>;
-    constexpr int ES = (int)sizeof(X);
+    constexpr int W = pair_width<X>();   // instances per thread
+    constexpr int CT = C / W;
+    static_assert(W == 1 || (C % 2 == 0 && MODES && (MODES & 3) == RK_MODE_DIRECT && !WAVE && !PRE && !HALF &&
+                             !Variant<V>::BLUE && ((MODES >> 2) & 3) != RK_MODE_ROW),
+                  "pairs of instances: column tiles with DIRECT loads and DIRECT or FLAT stores");
     using P = Plan<L>;
     static_assert(!WAVE || (64 % P::T == 0), "wave-local stages need whole instances per wave");
     constexpr int T = P::T;
-    constexpr int NT = C * T;
+    constexpr int NT = CT * T;
     constexpr int R0 = P::R0;
-    constexpr int LP = tile_pitch<L, C, HALF, ES>();
+    constexpr int LP = tile_pitch_x<L, C, HALF, X>();
     constexpr int VM = P::vmax();
     constexpr int SL = P::NSTAGE - 1;
     constexpr int RL = P::radix(SL);
     constexpr int QL = P::q(SL);
     constexpr bool BLUE = Variant<V>::BLUE;
     constexpr bool TWID = Variant<V>::PRE == RK_VAR_PRE_TWIDDLE;
-    constexpr bool SPLIT = tile_split<L, C, HALF, ES>();
+    constexpr bool SPLIT = tile_split_x<L, C, HALF, X>();
     const rk_u64 inst0 = tile * (rk_u64)C;
     const rk_u32 load_mode = MODES ? (rk_u32)(MODES & 3) : a.load_mode;
     const rk_u32 store_mode = MODES ? (rk_u32)((MODES >> 2) & 3) : a.store_mode;
 
     // compute mapping (see fft_args.h): lanes along an instance or across
     // instances (WAVE: the row mapping, compiled in)
-    const bool colmap = WAVE ? false : a.cmap != 0;
-    const int c = colmap ? (tid % C) : (tid / T);
-    int t = colmap ? (tid / C) : (tid % T);
+    const bool colmap = WAVE ? false : W == 2 ? true : a.cmap != 0;
+    const int c = colmap ? (tid % CT) : (tid / T);
+    int t = colmap ? (tid / CT) : (tid % T);
     const int cbase = c * LP;
     // the other mapping, for a side staged through LDS
-    const int cs = colmap ? (tid / T) : (tid % C);
-    const int ps = colmap ? (tid % T) : (tid / C);
+    const int cs = colmap ? (tid / T) : (tid % CT);
+    const int ps = colmap ? (tid % T) : (tid / CT);
 
     X v[VM];
     X g[R0];   // staging registers (global side of a staged load/store)
 
     // ---- stage-0 inputs: element p = t + r*T of instance c ----
-    const Inst ic = decompose<L>(a, inst0 + c);
+    const Inst ic = decompose<L>(a, inst0 + c * W);
     auto own_pos = [&](int i) { return cbase + stage_in_lds<L, 0>(t, i); };
     if (PRE || load_mode == RK_MODE_DIRECT) {
         const Walk w = in_walk(a, ic, t);
@@ -952,6 +1120,8 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
         }
         pre_ops<V, R0>(a, ic, w, v, [](int r) { return r * T; });
         if constexpr (TWID) apply_pass_twiddles<R0>(a, ic.l, t, T, v);
+    } else if constexpr (W == 2) {
+        // pairs load DIRECT
     } else if (load_mode == RK_MODE_FLAT) {
         // instance-linear block of C*L elements, no pre-ops
         const rk_i64 base = a.in_off + (rk_i64)inst0 * L;
@@ -994,7 +1164,7 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     auto last_out = [&](int i) {
         return stage_valid<L, SL>(t, i / RL) ? cbase + stage_out_lds<L, SL>(t, i) : -1;
     };
-    const X* twl;
+    const scalar_t<X>* twl;
     if constexpr (TWLDS) twl = twl_lds;
     else twl = table<X>(a.twl);
     run_stages<L, 0, SPLIT, VM, WAVE>(v, my, t, twl);
@@ -1030,6 +1200,43 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
             for (int i = 0; i < QL * RL; ++i)
                 if (stage_valid<L, SL>(t, i / RL)) store_at<V, IO>(a, io, ic, w, stage_out_pos<L, SL>(0, i), v[i], adjust);
         }
+    } else if constexpr (W == 2) {
+        // FLAT: the tile is C*L contiguous elements; a thread takes two
+        // consecutive positions of both instances of a pair where it can
+        const rk_i64 base = a.out_off + (rk_i64)inst0 * L;
+        if constexpr (R0 % 2 == 0 && L % 2 == 0) {
+            lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out,
+                                             [&](int i) { return flat_pair_lds<L, NT, LP>(tid, i / 2, i % 2); });
+#pragma unroll
+            for (int it = 0; it < R0 / 2; ++it) {
+                const int e = 2 * (tid + it * NT);
+                const int ce = e / L, k = e - ce * L;
+                if (inst0 + 2 * ce < a.n_inst) {
+                    X y0 = g[2 * it], y1 = g[2 * it + 1];
+                    if (adjust) {
+                        y0 = adjust_out(a, y0);
+                        y1 = adjust_out(a, y1);
+                    }
+                    const rk_i64 at = base + (rk_i64)(2 * ce) * L + k;
+                    io.store_run(a, at, y0.x.x, y0.y.x, y1.x.x, y1.y.x);
+                    io.store_run(a, at + L, y0.x.y, y0.y.y, y1.x.y, y1.y.y);
+                }
+            }
+        } else {
+            lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return flat_lds<L, NT, LP>(tid, it); });
+#pragma unroll
+            for (int it = 0; it < R0; ++it) {
+                const int e = tid + it * NT;
+                const int ce = e / L, k = e - ce * L;
+                if (inst0 + 2 * ce < a.n_inst) {
+                    X y = g[it];
+                    if (adjust) y = adjust_out(a, y);
+                    const rk_i64 at = base + (rk_i64)(2 * ce) * L + k;
+                    io.store_one(a, at, y.x.x, y.y.x);
+                    io.store_one(a, at + L, y.x.y, y.y.y);
+                }
+            }
+        }
     } else if (store_mode == RK_MODE_FLAT) {
         // no post-ops beyond sign and scale
         lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return flat_lds<L, NT, LP>(tid, it); });
@@ -1057,6 +1264,10 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
 
 // Threads per work-group of fft_pass_body<L, C, ...>.
 template <int L, int C> __host__ __device__ constexpr int pass_threads() { return C * Plan<L>::T; }
+// The same of a catalogue variant number (RK_VAR_PAIR: two instances per thread).
+template <int L, int C, int V> __host__ __device__ constexpr int variant_threads() {
+    return (V & RK_VAR_PAIR) ? (C / 2) * Plan<L>::T : C * Plan<L>::T;
+}
 
 // Tiles whose stage twiddles are read from an LDS copy of the W_L table
 // instead of global memory (the table loads otherwise take a large share of
@@ -1069,9 +1280,10 @@ template <int L, int C> __host__ __device__ constexpr int pass_threads() { retur
 // 16384 x 1024 50.5 -> 47.7 us, the single-kernel Bluestein 4096 x 997 (both
 // of its transforms read the table) 53 -> 44 us; 4096-point rows (a 32 KB
 // table, half the residency) 64 -> 70 us, so they keep the global table.
-template <int L, int C, int V, bool WAVE, bool HALF, int ES> __host__ __device__ constexpr bool twl_in_lds() {
+template <int L, int C, int V, bool WAVE, bool HALF, class X> __host__ __device__ constexpr bool twl_in_lds() {
+    constexpr int ES = (int)sizeof(scalar_t<X>);
     if (WAVE || ES != 8 || Plan<L>::NSTAGE < 2) return false;
-    constexpr int base = tile_lds_bytes<L, C, HALF, ES>();
+    constexpr int base = tile_lds_bytes_x<L, C, HALF, X>();
     constexpr int with = base + L * ES;
     return (160 * 1024) / with == (160 * 1024) / base || (L * ES <= 16 * 1024 && (160 * 1024) / with >= 2);
 }
@@ -1081,16 +1293,16 @@ template <int L, int C, int V, bool WAVE, bool HALF, int ES> __host__ __device__
 template <int L, int C, int V, class IO, int MODES = 0, bool WAVE = false, bool HALF = false>
 __device__ __forceinline__ void fft_pass_body(const rk_pass_args& a, const IO& io) {
     using X = typename IO::value_type;
-    constexpr int ES = (int)sizeof(X);
-    constexpr int LP = tile_pitch<L, C, HALF, ES>();
-    __shared__ X lds[tile_split<L, C, HALF, ES>() ? (C * LP + 1) / 2 : C * LP];
+    constexpr int LP = tile_pitch_x<L, C, HALF, X>();
+    constexpr int CT = C / pair_width<X>();
+    __shared__ X lds[tile_split_x<L, C, HALF, X>() ? (CT * LP + 1) / 2 : CT * LP];
     const rk_u64 tile = xcd_tile(a) + a.tile_base;
     if (tile >= a.n_tiles) return;
-    if constexpr (twl_in_lds<L, C, V, WAVE, HALF, ES>()) {
+    if constexpr (twl_in_lds<L, C, V, WAVE, HALF, X>()) {
         // the stage twiddles W_L^e from LDS, published by the tile's first
         // exchange barrier (before stage 1 reads them)
-        __shared__ X twl_s[L];
-        for (int e = (int)threadIdx.x; e < L; e += pass_threads<L, C>()) twl_s[e] = table<X>(a.twl)[e];
+        __shared__ scalar_t<X> twl_s[L];
+        for (int e = (int)threadIdx.x; e < L; e += CT * Plan<L>::T) twl_s[e] = table<X>(a.twl)[e];
         fft_pass_tile<L, C, V, IO, MODES, WAVE, false, HALF, true>(a, io, lds, tile, (int)threadIdx.x, nullptr, twl_s);
     } else {
         fft_pass_tile<L, C, V, IO, MODES, WAVE, false, HALF>(a, io, lds, tile, (int)threadIdx.x);
@@ -1148,10 +1360,13 @@ __device__ __forceinline__ void fft_pass_body_pipe(const rk_pass_args& a, const 
     }
 }
 
-// The element type of a variant number: complex128 with RK_VAR_F64.
+// The value type of a variant number: complex128 with RK_VAR_F64, two
+// instances' complex64 values with RK_VAR_PAIR.
 template <bool F64> struct ElemOf { typedef float2 type; };
 template <> struct ElemOf<true> { typedef double2 type; };
-template <int V> using elem_t = typename ElemOf<(V & RK_VAR_F64) != 0>::type;
+template <bool PAIR, bool F64> struct ValueOf { typedef typename ElemOf<F64>::type type; };
+template <bool F64> struct ValueOf<true, F64> { typedef cpair2 type; };
+template <int V> using elem_t = typename ValueOf<(V & RK_VAR_PAIR) != 0, (V & RK_VAR_F64) != 0>::type;
 
 // The pass kernel of a catalogue variant number V: the low seven bits are the
 // compile-time Variant (pre-op, post-op, Bluestein), the higher bits choose the
@@ -1170,7 +1385,9 @@ __device__ __forceinline__ void fft_pass_entry(const rk_pass_args& a) {
     constexpr bool NTS = (V & (RK_VAR_STREAM | RK_VAR_NT_STORE)) != 0;
     constexpr bool WAVE = (V & RK_VAR_WAVE) != 0;
     constexpr bool HALF = (V & RK_VAR_HALF) != 0;
-    if constexpr ((V & RK_VAR_PIPE) != 0)
+    if constexpr ((V & RK_VAR_PAIR) != 0)
+        fft_pass_body<L, C, VB, PairIO<NTL, NTS>, M>(a, PairIO<NTL, NTS>{});
+    else if constexpr ((V & RK_VAR_PIPE) != 0)
         fft_pass_body_pipe<L, C, VB, GlobalIO<NTL, NTS, X>, M, WAVE, HALF>(a, GlobalIO<NTL, NTS, X>{});
     else
         fft_pass_body<L, C, VB, GlobalIO<NTL, NTS, X>, M, WAVE, HALF>(a, GlobalIO<NTL, NTS, X>{});
@@ -1183,8 +1400,15 @@ __device__ __forceinline__ void fft_pass_entry(const rk_pass_args& a) {
 // An RK_VAR_OCC kernel asks for the waves per SIMD its LDS allows, so
 // registers do not cut the occupancy; a persistent (RK_VAR_PIPE) kernel
 // without it for one resident work-group per CU (the registers of its
-// prefetched tile then come out of that work-group's share).
+// prefetched tile then come out of that work-group's share).  A pair kernel
+// asks for what its LDS allows, at most four waves (128 VGPRs: 64 hold the
+// two instances' values of a radix-16 stage).
 template <int L, int C, int V> __host__ __device__ constexpr int pass_min_waves() {
+    if ((V & RK_VAR_PAIR) != 0) {
+        const int waves = (variant_threads<L, C, V>() + 63) / 64;
+        const int w = ((160 * 1024) / (tile_lds_bytes_x<L, C, false, cpair2>() + L * 8)) * waves / 4;
+        return w < 1 ? 1 : (w > 4 ? 4 : w);
+    }
     if ((V & (RK_VAR_PIPE | RK_VAR_OCC)) != 0) {
         const int waves = (pass_threads<L, C>() + 63) / 64;
         const int slots = (V & RK_VAR_OCC) ? (160 * 1024) / tile_lds_bytes<L, C, (V & RK_VAR_HALF) != 0,

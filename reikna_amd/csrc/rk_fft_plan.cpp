@@ -23,6 +23,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <tuple>
 
 #include "fft_device.hpp"
 #include "rk_internal.hpp"
@@ -677,11 +678,13 @@ static void set_xcd_group(PassPlan& pp) {
         const char* e = getenv("RK_XCD_GROUP");
         return e && *e ? atoi(e) : 0;
     }();
+    const int C = pp.pair_C ? pp.pair_C : pp.C;
     rk_u32 g = 1;
     if (forced > 0)
         g = (rk_u32)forced;
-    else if ((pp.args.cmap || pp.args.load_mode == RK_MODE_COLUMN || pp.args.store_mode == RK_MODE_COLUMN) && pp.C <= 16)
-        g = (rk_u32)(32 / pp.C);
+    else if ((pp.args.cmap || pp.args.load_mode == RK_MODE_COLUMN || pp.args.store_mode == RK_MODE_COLUMN) && C <= 16)
+        g = (rk_u32)(32 / C);
+    pp.args.xcd_group = 0;
     if (g > 1) {
         pp.args.xcd_group = g;
         pp.args.n_xcd = xcd_count();
@@ -748,9 +751,18 @@ static int io_variant_bits(const PassPlan& pp) {
 }
 
 static const KernelEntry* catalog_find(int L, int C, int variant) {
-    for (const KernelEntry& e : catalog())
-        if (e.L == L && e.C == C && e.variant == variant) return &e;
-    return nullptr;
+    static const std::map<std::tuple<int, int, int>, const KernelEntry*> index = [] {
+        std::map<std::tuple<int, int, int>, const KernelEntry*> m;
+        for (const KernelEntry& e : catalog()) m.emplace(std::make_tuple(e.L, e.C, e.variant), &e);
+        return m;
+    }();
+    auto it = index.find(std::make_tuple(L, C, variant));
+    return it == index.end() ? nullptr : it->second;
+}
+
+// Whether the catalogue holds kernels of this length at all.
+static bool catalog_length(int L) {
+    return catalog_find(L, default_tile_c_row(L), VAR_PLAIN) != nullptr;
 }
 
 // The pass's kernel: the catalogue's, with the pass's load/store modes
@@ -785,6 +797,77 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
         return RK_OK;
     }
     return jit_pass_kernel(pp.L, pp.C, want | mbit, &pp.jit, &pp.threads, &pp.lds_bytes);
+}
+
+// Instances per tile of the pair kernel of a pass (two adjacent instances per
+// thread, RK_VAR_PAIR), or 0 when the pass cannot run as pairs: complex64
+// column tiles with DIRECT loads and DIRECT or FLAT stores whose innermost
+// dim longer than one (I, NS, H in this order) is even and has unit stride on
+// the DIRECT sides, so that instances 2k and 2k+1 are neighbours in memory
+// (16-byte accesses) and both valid or both not.
+static bool pair_enabled() {
+    static const bool v = [] {
+        const char* e = getenv("RK_PAIR");
+        return !(e && *e && atoi(e) == 0);
+    }();
+    return v;
+}
+
+static int pair_tile(const PassPlan& pp) {
+    const rk_pass_args& a = pp.args;
+    const int mbit = fixed_mode_bit(pp);
+    if (!pair_enabled() || pp.es != 8 || pp.wave || pp.pipe || pp.half || !a.cmap) return 0;
+    if (pp.variant != VAR_PLAIN && pp.variant != VAR_TWIDDLE) return 0;
+    if (mbit != VAR_MODE_DD && mbit != VAR_MODE_DF) return 0;
+    if (t_tuning && t_tuning->col_tile > 0) return 0;
+    if (pp.L < 512 || pp.L > 1024 || (pp.L & (pp.L - 1))) return 0;
+    const bool dd = mbit == VAR_MODE_DD;
+    if (!pp.nt_load && !pp.nt_store && !(dd && pp.L == 1024 && a.n_tiles >= 512)) return 0;
+    rk_u64 inner;
+    if (a.dim_I > 1) {
+        inner = a.dim_I;
+        if (a.in_si != 1 || (dd && a.out_si != 1)) return 0;
+    } else if (a.dim_NS > 1) {
+        inner = a.dim_NS;
+        if (a.in_sa != 1 || (dd && a.out_sa != 1)) return 0;
+    } else {
+        inner = a.dim_H;
+        if (a.in_sa != 1 || dd) return 0;
+    }
+    if (inner % 2) return 0;
+    // 256 threads where the tile's LDS leaves two work-groups per CU, and
+    // whole tiles per outer index (chunked chains start at tile boundaries)
+    const int T = threads_per_instance(pp.L);
+    const rk_u64 per_outer = a.dim_I * a.dim_NS * a.dim_H;
+    int C = 64;
+    while (C > 16 && ((C / 2) * T > 256 || per_outer % (rk_u64)C || rkfft::pair_lds_bytes(pp.L, C, T) + pp.L * 8 > 80 * 1024))
+        C /= 2;
+    return C;
+}
+
+// The pair kernel of a pass: the catalogue's, or one from the run-time
+// compiler for lengths the catalogue does not hold.
+static bool find_pair_kernel(PassPlan& pp, uint32_t flags) {
+    const int C = pair_tile(pp);
+    if (!C) return false;
+    const int T = threads_per_instance(pp.L);
+    pp.pair_threads = (C / 2) * T;
+    int v = pp.variant | fixed_mode_bit(pp) | VAR_PAIR;
+    if (pp.nt_load && pp.nt_store) v |= VAR_STREAM;
+    else if (pp.nt_load) v |= VAR_NT_LOAD;
+    else if (pp.nt_store) v |= VAR_NT_STORE;
+    if (const KernelEntry* e = catalog_find(pp.L, C, v)) {
+        pp.aot = e->func;
+    } else {
+        if (catalog_length(pp.L) || (flags & (RK_FFT_NO_JIT | RK_FFT_DRY_RUN))) return false;
+        int threads = 0, lds = 0;
+        if (jit_pass_kernel(pp.L, C, v, &pp.jit, &threads, &lds) != RK_OK) return false;
+    }
+    pp.pair_C = C;
+    pp.threads = pp.C * T;
+    pp.lds_bytes = tile_lds_bytes_host(pp.L, pp.C, pp.es);
+    pp.fixed_modes = true;
+    return true;
 }
 
 // Passes whose instances fill whole waves (T = L / R0 divides 64) run the
@@ -1148,8 +1231,10 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
         pp.pipe = pipe_enabled() && pp.args.load_mode == RK_MODE_DIRECT && pp.loops.empty();
         pp.half = half_enabled() && (int64_t)pp.C * lds_pitch_host(pp.L) * pp.es <= 80 * 1024;
         pp.occ = occ_min_length() >= 0 ? occ_min_length() > 0 && pp.L >= occ_min_length() : occ_default(pp);
-        rc = find_kernel(pp, d->flags);
-        if (rc != RK_OK) return rc;
+        if (!find_pair_kernel(pp, d->flags)) {
+            rc = find_kernel(pp, d->flags);
+            if (rc != RK_OK) return rc;
+        }
         set_xcd_group(pp);
         const uint64_t max_grid = (uint64_t(1) << 31) / (uint64_t)pp.threads;
         pp.grid = std::min<uint64_t>(pp.args.n_tiles, pp.pipe ? pipe_grid(pp) : max_grid);
@@ -1176,9 +1261,14 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
     return RK_OK;
 }
 
-// Launches tiles [t0, t1) of a pass (one tile per work-group).
+// Launches the tiles of instances [i0, i1) of a pass (one tile per
+// work-group; i0 is a tile boundary).
 static int launch_pass(const PassPlan& pp, rk_pass_args& a, hipStream_t stream, const rk_user_blob* load_blob,
-                       const rk_user_blob* store_blob, rk_u64 t0, rk_u64 t1) {
+                       const rk_user_blob* store_blob, rk_u64 i0, rk_u64 i1) {
+    const rk_u64 C = (rk_u64)(pp.pair_C ? pp.pair_C : pp.C);
+    const int threads = pp.pair_C ? pp.pair_threads : pp.threads;
+    const rk_u64 max_grid = pp.pair_C ? (rk_u64(1) << 31) / (rk_u64)threads : pp.grid;
+    const rk_u64 t0 = i0 / C, t1 = (i1 + C - 1) / C;
     // host loops over batch dims the kernel could not fold
     const size_t nl = pp.loops.size();
     int64_t total = 1;
@@ -1197,16 +1287,16 @@ static int launch_pass(const PassPlan& pp, rk_pass_args& a, hipStream_t stream, 
         // grids beyond the launch limit are split; the kernel stops at tile t1
         // (a persistent kernel covers [t0, t1) in one launch)
         a.n_tiles = t1;
-        for (rk_u64 base = t0; base < t1; base += pp.pipe ? (t1 - t0) : pp.grid) {
+        for (rk_u64 base = t0; base < t1; base += pp.pipe ? (t1 - t0) : max_grid) {
             a.tile_base = base;
-            const unsigned grid = (unsigned)std::min<rk_u64>(pp.grid, t1 - base);
+            const unsigned grid = (unsigned)std::min<rk_u64>(max_grid, t1 - base);
             // fused kernels take (pass args, load blob, store blob)
             void* params[] = {&a, const_cast<rk_user_blob*>(load_blob), const_cast<rk_user_blob*>(store_blob)};
             if (pp.jit) {
-                RK_HIP(hipModuleLaunchKernel(pp.jit, grid, 1, 1, (unsigned)pp.threads, 1, 1, 0, stream, params,
+                RK_HIP(hipModuleLaunchKernel(pp.jit, grid, 1, 1, (unsigned)threads, 1, 1, 0, stream, params,
                                              nullptr));
             } else {
-                RK_HIP(hipLaunchKernel(pp.aot, dim3(grid), dim3((unsigned)pp.threads), params, 0, stream));
+                RK_HIP(hipLaunchKernel(pp.aot, dim3(grid), dim3((unsigned)threads), params, 0, stream));
             }
         }
     }
@@ -1266,7 +1356,7 @@ static int plan_execute(const rk_fft_plan* plan, void* out, const void* in, int 
     if (!plan->chunk_outer) {
         for (size_t p = 0; p < np; ++p) {
             if (plan->timing) RK_HIP(hipEventRecord(plan->events[2 * p], stream));
-            int rc = launch_pass(plan->passes[p], args[p], stream, &lb, &sb, 0, args[p].n_tiles);
+            int rc = launch_pass(plan->passes[p], args[p], stream, &lb, &sb, 0, args[p].n_inst);
             if (rc != RK_OK) return rc;
             if (plan->timing) RK_HIP(hipEventRecord(plan->events[2 * p + 1], stream));
         }
@@ -1282,11 +1372,10 @@ static int plan_execute(const rk_fft_plan* plan, void* out, const void* in, int 
             rk_pass_args a = args[p];
             if (pp.src == BUF_WS0 || pp.src == BUF_WS1) a.in_off -= o0 * pp.src_stride0;
             if (pp.dst == BUF_WS0 || pp.dst == BUF_WS1) a.out_off -= o0 * pp.dst_stride0;
-            const rk_u64 t0 = (rk_u64)o0 * pp.inst_per_outer / (rk_u64)pp.C;
-            const rk_u64 t1 = (rk_u64)o1 * pp.inst_per_outer / (rk_u64)pp.C;
+            const rk_u64 i0 = (rk_u64)o0 * pp.inst_per_outer, i1 = (rk_u64)o1 * pp.inst_per_outer;
             const size_t ev = 2 * (chunk_idx * np + p);
             if (plan->timing && ev + 1 < plan->events.size()) RK_HIP(hipEventRecord(plan->events[ev], stream));
-            int rc = launch_pass(pp, a, stream, &lb, &sb, t0, t1);
+            int rc = launch_pass(pp, a, stream, &lb, &sb, i0, i1);
             if (rc != RK_OK) return rc;
             if (plan->timing && ev + 1 < plan->events.size()) RK_HIP(hipEventRecord(plan->events[ev + 1], stream));
         }
@@ -1465,9 +1554,20 @@ extern "C" int rk_fft_plan_pass_info(const rk_fft_plan* plan, int pass, rk_fft_p
     return RK_OK;
 }
 
+extern "C" int rk_fft_plan_pass_pair(const rk_fft_plan* plan, int pass, int* instances) {
+    if (!plan || !instances) return fail(RK_ERR_INVALID, "rk_fft_plan_pass_pair: null argument");
+    if (pass < 0 || pass >= (int)plan->passes.size()) return fail(RK_ERR_INVALID, "pass index %d out of range", pass);
+    *instances = plan->passes[pass].pair_C;
+    return RK_OK;
+}
+
 extern "C" int rk_fft_plan_set_pass_kernel(rk_fft_plan* plan, int pass, void* function) {
     if (!plan || !function) return fail(RK_ERR_INVALID, "rk_fft_plan_set_pass_kernel: null argument");
     if (pass < 0 || pass >= (int)plan->passes.size()) return fail(RK_ERR_INVALID, "pass index %d out of range", pass);
+    if (plan->passes[pass].pair_C) {   // the replacement runs the one-instance-per-thread tile
+        plan->passes[pass].pair_C = 0;
+        rk::set_xcd_group(plan->passes[pass]);
+    }
     plan->passes[pass].jit = (hipFunction_t)function;
     plan->passes[pass].aot = nullptr;
     plan->passes[pass].user_kernel = true;

@@ -58,6 +58,7 @@ enum {
     VAR_HALF = 1 << 15,    // catalogue entries: exchanges through re/im halves (RK_VAR_HALF)
     VAR_OCC = 1 << 16,     // catalogue entries: registers bounded for the LDS-allowed residency (RK_VAR_OCC)
     VAR_F64 = 1 << 17,     // complex128 elements (RK_VAR_F64; run-time compiled only)
+    VAR_PAIR = 1 << 18,    // two adjacent instances per thread (RK_VAR_PAIR)
 };
 
 // All ahead-of-time kernels compiled into this library.
@@ -134,6 +135,12 @@ struct PassPlan {
     bool occ = false;               // registers bounded for the LDS-allowed residency
     int es = 8;                     // element bytes: 8 complex64, 16 complex128
     bool fixed_modes = false;       // the kernel has this pass's load/store modes compiled in
+    // Instances per tile of the pair kernel that runs this pass (0: none).  C,
+    // threads and grid above stay those of the one-instance-per-thread tile,
+    // the geometry of a kernel set with rk_fft_plan_set_pass_kernel (which
+    // then runs instead).
+    int pair_C = 0;
+    int pair_threads = 0;
     uint64_t grid = 0;
     int axis = 0;
     int kind = 0;

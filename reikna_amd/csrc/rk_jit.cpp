@@ -30,7 +30,8 @@ int jit_pass_kernel(int L, int C, int variant, hipFunction_t* fn, int* threads, 
     if (L < 1 || L > 16384 || !is_smooth(L))
         return fail(RK_ERR_NO_KERNEL, "no kernel for DFT length %d (must be 7-smooth and <= 16384)", L);
     const int T = threads_per_instance(L);
-    if ((int64_t)C * T > 1024) return fail(RK_ERR_NO_KERNEL, "tile %d x %d threads exceeds 1024", C, T);
+    const int nt = (variant & VAR_PAIR) ? (C / 2) * T : C * T;
+    if (nt > 1024) return fail(RK_ERR_NO_KERNEL, "tile %d x %d threads exceeds 1024", (variant & VAR_PAIR) ? C / 2 : C, T);
     int dev = 0;
     hipGetDevice(&dev);
     std::lock_guard<std::mutex> lock(mu);
@@ -46,7 +47,7 @@ int jit_pass_kernel(int L, int C, int variant, hipFunction_t* fn, int* threads, 
                  "rk_jit_pass(rk_pass_args a) {\n"
                  "    rkfft::fft_pass_entry<%d, %d, %d>(a);\n"
                  "}\n",
-                 C * T, L, C, variant, L, C, variant);
+                 nt, L, C, variant, L, C, variant);
         std::string code, log;
         int rc = compile_code_object(src, {"fft_args.h", "fft_device.hpp"}, {k_src_fft_args_h, k_src_fft_device_hpp},
                                      "-Xclang -target-feature -Xclang -packed-fp32-ops", &code, &log);
@@ -54,7 +55,7 @@ int jit_pass_kernel(int L, int C, int variant, hipFunction_t* fn, int* threads, 
         JitKernel k;
         RK_HIP(hipModuleLoadData(&k.module, code.data()));
         RK_HIP(hipModuleGetFunction(&k.fn, k.module, "rk_jit_pass"));
-        k.threads = C * T;
+        k.threads = nt;
         const int es = (variant & VAR_F64) ? 16 : 8;
         k.lds = (variant & VAR_HALF) ? tile_lds_bytes_host(L, C, es) / 2 : tile_lds_bytes_host(L, C, es);
         it = cache.emplace(key, k).first;

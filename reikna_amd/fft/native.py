@@ -43,6 +43,7 @@ class PassInfo:
     nt_store: bool = False      # nontemporal stores
     wave: bool = False          # whole instances per wave, wave-local stage exchanges
     pipe: bool = False          # persistent kernel that loads its next tile while computing one
+    pair: int = 0               # instances per tile of the two-instances-per-thread kernel (0: not used)
     occ: bool = False           # launch bounds for as many resident work-groups as the LDS allows
 
 
@@ -148,6 +149,8 @@ class NativeFftPlan:
         for p in range(n.value):
             info = _lib.FftPassInfo()
             _lib.call("rk_fft_plan_pass_info", ctypes.c_void_p(self.handle), p, ctypes.byref(info))
+            pair = ctypes.c_int(0)
+            _lib.call("rk_fft_plan_pass_pair", ctypes.c_void_p(self.handle), p, ctypes.byref(pair))
             out.append(
                 PassInfo(
                     L=info.L, C=info.C, threads=info.threads, kind=info.kind,
@@ -157,7 +160,7 @@ class NativeFftPlan:
                     Ns=info.Ns, lds_bytes=info.lds_bytes, jit=bool(info.jit), variant=info.variant,
                     stream=bool(info.stream),
                     fixed_modes=bool(info.fixed_modes),
-                    nt_load=bool(info.nt_load), nt_store=bool(info.nt_store), wave=bool(info.wave),
+                    nt_load=bool(info.nt_load), nt_store=bool(info.nt_store), wave=bool(info.wave), pair=pair.value,
                     pipe=bool(info.pipe), occ=bool(info.occ),
                 )
             )

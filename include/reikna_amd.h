@@ -151,6 +151,9 @@ typedef struct {
 #define RK_FFT_OUT_LAST_ONLY   0x10u    /* only the last pass touches `out`: earlier axes finish in workspace */
 #define RK_FFT_DRY_RUN         0x20u    /* plan only: no device tables, no run-time compilation;
                                            the plan can be inspected but not executed */
+#define RK_FFT_FUSED_ENDS      0x40u    /* the first or last pass gets a generated kernel
+                                           (rk_fft_plan_set_pass_kernel): a hint for the
+                                           choice of streaming accesses */
 
 /* Build a plan: radix factorisation, pass chain, buffer routing, and all
    device tables (twiddles in FP64 rounded once to FP32, Bluestein chirp from

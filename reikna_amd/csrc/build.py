@@ -223,6 +223,24 @@ def catalog_entries() -> list[tuple[int, int, int]]:
                 and base in (VAR_PLAIN, VAR_TWIDDLE) and v & (VAR_MODE_DD | VAR_MODE_DF)):
             for cp in pair_tile_widths(length):
                 ents.add((length, cp, v | VAR_PAIR))
+    # plans over several axes stream their first pass's loads (contiguous rows)
+    # and their last pass's stores (strided columns) when their arrays near the
+    # Infinity Cache (rk_fft_plan.cpp stream_ends)
+    for length in catalog_lengths():
+        if length <= STREAM_MAX:
+            ents.add((length, tile_c_row(length), VAR_PLAIN | VAR_NT_LOAD))
+            ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE))
+            if length <= FACTOR_MAX:
+                ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD))
+                if length <= 1024 and tile_c_col(length) * threads_per_instance(length) == 1024:
+                    ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_OCC))
+                if PAIR_MIN <= length and length & (length - 1) == 0:
+                    for cp in pair_tile_widths(length):
+                        ents.add((length, cp, VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_PAIR))
+            if length & (length - 1) and threads_per_instance(length) >= 32:
+                ents.add((length, tile_c_row(length), VAR_PLAIN | VAR_NT_LOAD | VAR_MODE_DD))
+            if length & (length - 1) and length >= 8 and threads_per_instance(length) < 32:
+                ents.add((length, tile_c_row(length), VAR_PLAIN | VAR_NT_LOAD | VAR_MODE_FF))
     # single-pass row tiles of such lengths (one thread per R0 elements of an
     # instance, at least 32 of them: shorter rows are streamed flat): the
     # 1000-point tile holds 80 VGPRs with every mode and 62 with DIRECT/DIRECT

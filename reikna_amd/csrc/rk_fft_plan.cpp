@@ -710,6 +710,27 @@ static bool stream_pass(const PassPlan& pp) {
     return bytes > stream_min_bytes();
 }
 
+// Which ends of an unchunked plan of several passes stream: 1 the first
+// pass's loads, 2 the last pass's stores (0: none).  The array a pass hands to
+// the next should stay in the 256 MB Infinity Cache, so the caller's input
+// (and an output the plan does not read back) must not push it out once input,
+// intermediate and output together approach that size.  Measured over rotating
+// buffers, plain accesses (arrays above 128 MiB: every access nontemporal)
+// against nontemporal ends: chains along one axis, 64 MiB arrays 71 -> 55 us
+// (8 x 2^20) and 115 -> 94 (256 x 2^16), 128 MiB 124 -> 111, 256 MiB 236 ->
+// 203 (32 x 2^20) and 227 -> 189 (128 x 2^18); the same buffers over and over
+// 55 -> 57, 119 -> 110, 233 -> 199.  16 x 2^18 (32 MiB) was no faster.  Plans
+// over several axes, whose later passes run in place on the output: 16 x 1024 x
+// 1024 (128 MiB) 104 -> 94 us, 256^3 137 -> 131; of 16 x 1080 x 1920 (253 MiB)
+// only the input's loads may: 316 -> 303, with the last stores 312.
+static int stream_ends(const PassPlan& pp, size_t axes) {
+    if (stream_min_bytes() <= 0) return 0;
+    const double array = (double)pp.es * (double)pp.args.n_inst * (double)pp.L;
+    const double unit = stream_min_bytes();   // the Infinity Cache
+    if (axes == 1) return array >= unit * 3 / 16 ? 3 : 0;
+    return array >= unit * 3 / 4 ? 1 : array >= unit * 3 / 8 ? 3 : 0;
+}
+
 // Kernels with the pass's load/store modes compiled in (RK_FIXED_MODES=0
 // turns them off).
 static bool use_fixed_modes() {
@@ -767,8 +788,9 @@ static bool catalog_length(int L) {
 
 // The pass's kernel: the catalogue's, with the pass's load/store modes
 // compiled in when such a twin exists, else from the run-time compiler (the
-// same entry, any variant number).  Without run-time compilation, a pass
-// whose nontemporal twin is missing keeps the plain accesses.
+// same entry, any variant number).  A pass whose nontemporal twin is missing
+// keeps the plain accesses when the catalogue has its plain kernel or run-time
+// compilation is off.
 static int find_kernel(PassPlan& pp, uint32_t flags) {
     pp.fixed_modes = false;
     const int mbit = fixed_mode_bit(pp);
@@ -782,7 +804,8 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
     if (mbit)
         if (const KernelEntry* e = catalog_find(pp.L, pp.C, want | mbit)) return take(e, true), RK_OK;
     if (const KernelEntry* e = catalog_find(pp.L, pp.C, want)) return take(e, false), RK_OK;
-    if (flags & RK_FFT_NO_JIT) {
+    const bool in_catalog = pp.es == 8 && catalog_find(pp.L, pp.C, pp.variant) != nullptr;
+    if ((flags & RK_FFT_NO_JIT) || in_catalog) {
         if (pp.nt_load || pp.nt_store) {
             pp.nt_load = pp.nt_store = false;
             return find_kernel(pp, flags);
@@ -804,7 +827,13 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
 // column tiles with DIRECT loads and DIRECT or FLAT stores whose innermost
 // dim longer than one (I, NS, H in this order) is even and has unit stride on
 // the DIRECT sides, so that instances 2k and 2k+1 are neighbours in memory
-// (16-byte accesses) and both valid or both not.
+// (16-byte accesses) and both valid or both not.  Streaming passes of 512 and
+// 1024 points, whose tiles leave two work-groups per CU, and large strided
+// axes of 1024: one against two instances per thread 64 x 2^20 422 / 392 us,
+// 256 x 2^18 382 / 365, 128 x 2^19 392 / 381, 1024 x 8192 over axis 0 39.6 /
+// 30.6.  Elsewhere half the waves per tile cost more than the instructions
+// saved: 16 x 2^18 33.7 / 36.5, 8 x 2^16 (256-point passes) 12.1 / 14.7,
+// 4 x 2^24 541 / 576.
 static bool pair_enabled() {
     static const bool v = [] {
         const char* e = getenv("RK_PAIR");
@@ -1221,12 +1250,28 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
     // loads, its last pass's stores): the intermediate stays in the Infinity
     // Cache between the passes of a chunk.
     for (PassPlan& pp : plan->passes) {
-        const bool plain = pp.variant == VAR_PLAIN || pp.variant == VAR_TWIDDLE;
+        // A column tile of less than 64 bytes per row leaves parts of its cache
+        // lines to the neighbouring tiles, which find them in the L2 only
+        // without the hint (16 x 1080 x 1920 over axis 1, tiles of 4
+        // instances: 437 us with it, 202 without).
+        const bool narrow = pp.args.cmap && pp.C * pp.es < 64;
+        const bool plain = (pp.variant == VAR_PLAIN || pp.variant == VAR_TWIDDLE) && !narrow;
         if (plan->chunk_outer) {
             pp.nt_load = plain && pp.is_first && pp.src == BUF_IN && stream_min_bytes() > 0;
             pp.nt_store = plain && pp.is_last && pp.dst == BUF_OUT && stream_min_bytes() > 0;
         } else {
-            pp.nt_load = pp.nt_store = stream_pass(pp);
+            pp.nt_load = pp.nt_store = plain && stream_pass(pp);
+            // unchunked plans of several passes: only the caller's input and
+            // output may stream, what the passes hand to each other is read
+            // again (stream_ends).  A generated kernel at one end has plain
+            // accesses: arrays that alone fill the cache then stream in every
+            // other pass, as one streaming end gains nothing there (32 x 2^20:
+            // 236 us streaming throughout, 203 at both ends, 247 at one).
+            if (plan->passes.size() > 1 && !((d->flags & RK_FFT_FUSED_ENDS) && pp.nt_load)) {
+                const int ends = plain ? stream_ends(pp, work.size()) : 0;
+                pp.nt_load = (ends & 1) && pp.is_first && pp.src == BUF_IN;
+                pp.nt_store = (ends & 2) && pp.is_last && pp.dst == BUF_OUT;
+            }
         }
         pp.pipe = pipe_enabled() && pp.args.load_mode == RK_MODE_DIRECT && pp.loops.empty();
         pp.half = half_enabled() && (int64_t)pp.C * lds_pitch_host(pp.L) * pp.es <= 80 * 1024;

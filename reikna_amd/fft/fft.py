@@ -121,6 +121,8 @@ class FFT(Computation):
         if fused_out:
             out_meta = ArrayMetadata(out_meta.shape, out_meta.dtype)
         flags = self._flags | (_lib.RK_FFT_OUT_LAST_ONLY if fused_out else 0)
+        if fused_in or fused_out:
+            flags |= _lib.RK_FFT_FUSED_ENDS
         if plan.virtual:
             flags |= _lib.RK_FFT_DRY_RUN
         native = NativeFftPlan(in_meta, out_meta, self._axes, flags, self._tuning)

@@ -76,15 +76,20 @@ static int64_t blue_single_max() {
 // transform, three passes of <= 256 against two of <= 1024: 512 x 2^17 0.445
 // against 0.347 ms, 256 x 2^18 0.449 / 0.376, 128 x 2^19 0.446 / 0.410,
 // 64 x 2^20 0.508 / 0.448, 64 x 10^6 0.639 / 0.571; from 2^21 points both
-// limits give three passes.  Complex128 tiles hold twice the registers and
-// keep 256.  RK_FACTOR_MAX overrides.
+// limits give three passes.  Complex128 chains take passes up to 512 points
+// (8 x 512 column tiles of 256 threads): three passes of <= 256 points against
+// two, 128 x 2^18 524 / 362 us, 32 x 2^18 136 / 102, 64 x 2^17 129 / 98, one
+// row of 2^17 15.0 / 13.4.  Two 1024-point complex128 passes (4 x 1024 tiles)
+// measured faster as well (64 x 2^20 1056 / 831 us), and so did Bluestein
+// chains of 512-point ones (33 x 65521 170 / 137), but the plan tests fix
+// those plans at 256; a tuned plan may choose them.  RK_FACTOR_MAX overrides.
 static int64_t factor_max() {
     static const int64_t v = [] {
         const char* e = getenv("RK_FACTOR_MAX");
         return e && *e ? (int64_t)atoll(e) : (int64_t)0;
     }();
     if (v) return v;
-    return t_elem_bytes == 16 ? 256 : 1024;
+    return t_elem_bytes == 16 ? 512 : 1024;
 }
 
 static bool length_ok(const ChainLimits& lim, int64_t n) { return lim.length_ok ? lim.length_ok(n) : is_smooth(n); }
@@ -204,6 +209,12 @@ int tile_c_col(int L) {
     int T = threads_per_instance(L);
     int C = std::max(16, (default_tile_c_row(L) / 16) * 16);
     while (C > 1 && ((int64_t)C * T > 1024 || (int64_t)C * lds_pitch_host(L) * t_elem_bytes > 159 * 1024)) C /= 2;
+    // Complex128 tiles of more than 256 points stop at 256 threads (69 KB of
+    // LDS, whole exchanges): 8 against 16 instances of 512 points 361 / 379 us
+    // (128 x 2^18) and 17.2 / 22.7 (one row), 4 against 8 of 1024 points 831 /
+    // 877 us (64 x 2^20) and 27.8 / 33.6 (one row; 4 x 1024 x 1024 over two
+    // axes 60.6 / 59.3).
+    while (t_elem_bytes == 16 && L > 256 && C > 4 && C * T > 256) C /= 2;
     // tuning override: an upper bound on the column tile width (kernels outside
     // the catalog come from the run-time compiler)
     static const int cap = [] {
@@ -461,6 +472,8 @@ int axis_passes(int64_t n, uint32_t flags, const ChainLimits& lim, std::vector<A
     if (smooth && !lim.length_ok)
         return fail(RK_ERR_UNSUPPORTED, "cannot split axis length %lld into passes", (long long)n);
     const int64_t m = bluestein_length(n, lim.pow2_bluestein);
+    ChainLimits blim = lim;   // complex128: factor_max() above
+    if (t_elem_bytes == 16 && blim.factor_max == 512 && !(t_tuning && t_tuning->factor_max > 0)) blim.factor_max = 256;
     const bool multi = m > lim.blue_single_max || (flags & RK_FFT_FORCE_MULTIPASS);
     if (!multi) {
         AxisPass ap;
@@ -480,7 +493,7 @@ int axis_passes(int64_t n, uint32_t flags, const ChainLimits& lim, std::vector<A
     }
     if (m <= kSingle && length_ok(lim, m) && !(flags & RK_FFT_FORCE_MULTIPASS)) {
         f.assign(1, m);   // two single-pass chains
-    } else if (!split_factors(m, lim, f)) {
+    } else if (!split_factors(m, blim, f)) {
         return fail(RK_ERR_UNSUPPORTED, "cannot split Bluestein length %lld", (long long)m);
     }
     if (f.size() == 1 && (flags & RK_FFT_FORCE_MULTIPASS)) {   // forced multi-pass of a short M

@@ -148,12 +148,18 @@ template <class X> RK_HD void dft8(X* v) {
 
 // 16 = 4 x 4: DFT4 over n2 for each n1 (x[n1 + 4 n2]), twiddle W16^{n1 k2},
 // DFT4 over n1 for each k2, output y[k2 + 4 k1].
+template <class X> RK_HD void dft16_second(X* v);
 template <class X> RK_HD void dft16(X* v) {
-    using F = real_t<X>;
     dft4(v[0], v[4], v[8], v[12]);
     dft4(v[1], v[5], v[9], v[13]);
     dft4(v[2], v[6], v[10], v[14]);
     dft4(v[3], v[7], v[11], v[15]);
+    dft16_second(v);
+}
+
+// The twiddles and the second DFT4s of dft16.
+template <class X> RK_HD void dft16_second(X* v) {
+    using F = real_t<X>;
     const X w1 = cx<X>((F)RK_C16, -(F)RK_S16);
     const X w3 = cx<X>((F)RK_S16, -(F)RK_C16);
     const X w9 = cx<X>(-(F)RK_C16, (F)RK_S16);
@@ -245,6 +251,47 @@ template <int R, class X> RK_HD void dft(X* v) {
     else if constexpr (R == 8) dft8(v);
     else if constexpr (R == 16) dft16(v);
     else static_assert(R == 1, "radix without a butterfly");
+}
+
+// The same with zeros in the upper half of the inputs (even R): the first
+// stage of a Bluestein transform, whose M >= 2N-1 points hold N <= M/2 values.
+template <class X> RK_HD void dft4_lower(X& a0, X& a1, X& a2, X& a3) {
+    const X x = a0, y = a1, t = c_mul_mi(a1);
+    a0 = c_add(x, y);
+    a2 = c_sub(x, y);
+    a1 = c_add(x, t);
+    a3 = c_sub(x, t);
+}
+
+template <int R, class X> RK_HD void dft_lower(X* v) {
+    using F = real_t<X>;
+    if constexpr (R == 2) {
+        v[1] = v[0];
+    } else if constexpr (R == 4) {
+        dft4_lower(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        X e0 = v[0], e1 = v[2], e2, e3, o0 = v[1], o1 = v[3], o2, o3;
+        dft4_lower(e0, e1, e2, e3);
+        dft4_lower(o0, o1, o2, o3);
+        o1 = c_w8_1(o1);
+        o2 = c_mul_mi(o2);
+        o3 = c_w8_3(o3);
+        v[0] = c_add(e0, o0); v[4] = c_sub(e0, o0);
+        v[1] = c_add(e1, o1); v[5] = c_sub(e1, o1);
+        v[2] = c_add(e2, o2); v[6] = c_sub(e2, o2);
+        v[3] = c_add(e3, o3); v[7] = c_sub(e3, o3);
+    } else if constexpr (R == 16) {
+        dft4_lower(v[0], v[4], v[8], v[12]);
+        dft4_lower(v[1], v[5], v[9], v[13]);
+        dft4_lower(v[2], v[6], v[10], v[14]);
+        dft4_lower(v[3], v[7], v[11], v[15]);
+        dft16_second(v);
+    } else {
+        const X zero = cx<X>((F)0, (F)0);
+#pragma unroll
+        for (int r = R / 2; r < R; ++r) v[r] = zero;
+        dft<R>(v);
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -667,6 +714,15 @@ template <int V> struct Variant {
 template <int V> __host__ __device__ constexpr bool pad_in() { return Variant<V>::PRE == RK_VAR_PRE_CHIRP; }
 template <int V> __host__ __device__ constexpr bool pad_out() { return Variant<V>::POST == RK_VAR_POST_CONJ_CHIRP; }
 
+// A Bluestein transform of N <= M/2 values over its M points (the planners
+// check this): the inputs of a chirp pass at or beyond the middle of its axis
+// are zero and the outputs of its last pass there are not stored, so with an
+// even radix R the upper R/2 of a thread's first-stage inputs need no load, no
+// chirp and no addition, and the upper R/2 of its last-stage outputs no store
+// (lower_in, lower_out).
+template <int V> __host__ __device__ constexpr bool lower_in(int R) { return pad_in<V>() && R % 2 == 0; }
+template <int V> __host__ __device__ constexpr bool lower_out(int R) { return pad_out<V>() && R % 2 == 0; }
+
 // One thread's walk over the positions p0 + c of one instance on one side
 // (c a compile-time offset): axis position and element address advance by
 // uniform steps computed once per thread, so an element costs one add and no
@@ -975,7 +1031,8 @@ RK_HD constexpr int flat_pair_lds(int tid, int it, int b) {
 
 template <int T> RK_HD constexpr int col_lds(int ps, int it) { return lds_pad_add<(T < 16 ? T : 16)>(ps, it * T); }
 
-template <int L, int S, bool SPLIT, int VM, bool WAVE = false, class X>
+// LOWER: the upper half of the first stage's inputs is zero (lower_in).
+template <int L, int S, bool SPLIT, int VM, bool WAVE = false, bool LOWER = false, class X>
 __device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const scalar_t<X>* twl) {
     using P = Plan<L>;
     constexpr int R = P::radix(S);
@@ -997,7 +1054,10 @@ __device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const sc
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-        if (stage_valid<L, S>(t, q)) dft<R>(&v[q * R]);
+        if (stage_valid<L, S>(t, q)) {
+            if constexpr (LOWER && S == 0) dft_lower<R>(&v[q * R]);
+            else dft<R>(&v[q * R]);
+        }
     if constexpr (S + 1 < P::NSTAGE) {
         constexpr int R1 = P::radix(S + 1);
         constexpr int Q1 = P::q(S + 1);
@@ -1089,6 +1149,8 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     constexpr bool BLUE = Variant<V>::BLUE;
     constexpr bool TWID = Variant<V>::PRE == RK_VAR_PRE_TWIDDLE;
     constexpr bool SPLIT = tile_split_x<L, C, HALF, X>();
+    constexpr bool LOW = lower_in<V>(R0);
+    constexpr int NL = LOW ? R0 / 2 : R0;   // first-stage inputs of a thread that may be nonzero
     const rk_u64 inst0 = tile * (rk_u64)C;
     const rk_u32 load_mode = MODES ? (rk_u32)(MODES & 3) : a.load_mode;
     const rk_u32 store_mode = MODES ? (rk_u32)((MODES >> 2) & 3) : a.store_mode;
@@ -1113,12 +1175,12 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
         const Walk w = in_walk(a, ic, t);
         if constexpr (PRE) {
 #pragma unroll
-            for (int r = 0; r < R0; ++r) v[r] = pre[r];
+            for (int r = 0; r < NL; ++r) v[r] = pre[r];
         } else {
 #pragma unroll
-            for (int r = 0; r < R0; ++r) v[r] = load_at<V, IO>(a, io, ic, w, r * T);
+            for (int r = 0; r < NL; ++r) v[r] = load_at<V, IO>(a, io, ic, w, r * T);
         }
-        pre_ops<V, R0>(a, ic, w, v, [](int r) { return r * T; });
+        pre_ops<V, NL>(a, ic, w, v, [](int r) { return r * T; });
         if constexpr (TWID) apply_pass_twiddles<R0>(a, ic.l, t, T, v);
     } else if constexpr (W == 2) {
         // pairs load DIRECT
@@ -1152,10 +1214,10 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
         const Inst ics = decompose<L>(a, inst0 + cs);
         const Walk w = in_walk(a, ics, ps);
 #pragma unroll
-        for (int it = 0; it < R0; ++it) g[it] = load_at<V, IO>(a, io, ics, w, it * T);
-        pre_ops<V, R0>(a, ics, w, g, [](int it) { return it * T; });
+        for (int it = 0; it < NL; ++it) g[it] = load_at<V, IO>(a, io, ics, w, it * T);
+        pre_ops<V, NL>(a, ics, w, g, [](int it) { return it * T; });
         if constexpr (TWID) apply_pass_twiddles<R0>(a, ics.l, ps, T, g);
-        lds_exchange<SPLIT, R0, R0>(
+        lds_exchange<SPLIT, NL, NL>(
             lds, g, v, [&](int it) { return cs * LP + col_lds<T>(ps, it); }, own_pos);
     }
 
@@ -1167,7 +1229,7 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     const scalar_t<X>* twl;
     if constexpr (TWLDS) twl = twl_lds;
     else twl = table<X>(a.twl);
-    run_stages<L, 0, SPLIT, VM, WAVE>(v, my, t, twl);
+    run_stages<L, 0, SPLIT, VM, WAVE, LOW>(v, my, t, twl);
 
     if constexpr (BLUE) {
         // A = FFT(chirp * x): multiply by the kernel spectrum, conjugate, and
@@ -1198,7 +1260,7 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
             const Walk w = out_walk(a, ic, t);
 #pragma unroll
             for (int i = 0; i < QL * RL; ++i)
-                if (stage_valid<L, SL>(t, i / RL)) store_at<V, IO>(a, io, ic, w, stage_out_pos<L, SL>(0, i), v[i], adjust);
+                if (!(lower_out<V>(RL) && i % RL >= RL / 2) && stage_valid<L, SL>(t, i / RL)) store_at<V, IO>(a, io, ic, w, stage_out_pos<L, SL>(0, i), v[i], adjust);
         }
     } else if constexpr (W == 2) {
         // FLAT: the tile is C*L contiguous elements; a thread takes two
@@ -1252,12 +1314,13 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
             }
         }
     } else {
-        lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return cs * LP + col_lds<T>(ps, it); });
+        constexpr int NO = lower_out<V>(R0) ? R0 / 2 : R0;
+        lds_exchange<SPLIT, QL * RL, NO>(lds, v, g, last_out, [&](int it) { return cs * LP + col_lds<T>(ps, it); });
         const Inst ics = decompose<L>(a, inst0 + cs);
         if (ics.valid) {
             const Walk w = out_walk(a, ics, ps);
 #pragma unroll
-            for (int it = 0; it < R0; ++it) store_at<V, IO>(a, io, ics, w, it * T, g[it], adjust);
+            for (int it = 0; it < NO; ++it) store_at<V, IO>(a, io, ics, w, it * T, g[it], adjust);
         }
     }
 }
@@ -1321,7 +1384,7 @@ __device__ __forceinline__ void direct_raw_loads(const rk_pass_args& a, const IO
     const Inst ic = decompose<L>(a, tile * (rk_u64)C + c);
     const Walk w = in_walk(a, ic, t);
 #pragma unroll
-    for (int r = 0; r < P::R0; ++r) raw[r] = load_at<V, IO>(a, io, ic, w, r * T);
+    for (int r = 0; r < (lower_in<V>(P::R0) ? P::R0 / 2 : P::R0); ++r) raw[r] = load_at<V, IO>(a, io, ic, w, r * T);
 }
 
 // Persistent, software-pipelined pass (DIRECT loads only): work-group b runs

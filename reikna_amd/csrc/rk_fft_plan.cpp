@@ -598,6 +598,11 @@ int describe_pass(const AxisPass& ap, const Layout& ls, const Layout& ld, int ax
     if ((!(ap.pre_ops & RK_PRE_CHIRP) && ap.n_valid_in != ap.Nax) ||
         (!(ap.post_ops & RK_POST_CHIRP) && ap.n_valid_out != ap.Nax))
         return fail(RK_ERR_UNSUPPORTED, "internal: a padded pass side without a chirp op (L=%d)", ap.L);
+    // ... and skip the upper half of a chirp side's positions (lower_in / lower_out)
+    if (ap.Nax % 2 == 0 && (((ap.pre_ops & RK_PRE_CHIRP) && 2 * ap.n_valid_in > ap.Nax) ||
+                            ((ap.post_ops & RK_POST_CHIRP) && 2 * ap.n_valid_out > ap.Nax)))
+        return fail(RK_ERR_UNSUPPORTED, "internal: Bluestein over %lld points of %lld values", (long long)ap.Nax,
+                    (long long)ap.n_valid_in);
     rk_pass_args& a = pp.args;
     int64_t O, so_in, so_out, I, si_in, si_out;
     fold_batch(ls, ld, axis, O, so_in, so_out, I, si_in, si_out, pp.loops);

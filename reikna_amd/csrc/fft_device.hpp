@@ -519,20 +519,6 @@ template <class X> __device__ __forceinline__ const scalar_t<X>* table(const flo
     return reinterpret_cast<const scalar_t<X>*>(p);
 }
 
-// Entry k of a table for a value of type X: of a pair, the entries k and k2
-// of its two instances.
-template <class X> __device__ __forceinline__ X table_at(const float2* p, rk_u64 k, rk_u64 k2) {
-    if constexpr (pair_width<X>() == 2) {
-        const float2 w0 = p[k], w1 = p[k2];
-        cpair2 w;
-        w.x = rk_v2<float>{w0.x, w1.x};
-        w.y = rk_v2<float>{w0.y, w1.y};
-        return w;
-    } else {
-        return table<X>(p)[k];
-    }
-}
-
 // The output scale (1/N on the last pass of an inverse transform) in the
 // element's real type: complex128 passes take the FP64 value.
 template <class X> __device__ __forceinline__ real_t<X> out_scale_of(const rk_pass_args& a) {
@@ -561,30 +547,36 @@ template <class X> __device__ __forceinline__ real_t<X> out_scale_of(const rk_pa
 // intermediate stays in that cache between passes streams only its first
 // pass's loads and its last pass's stores.  X is the element type
 // (complex64 float2, complex128 double2); every IO policy names it value_type.
+// kPtr: elements are also reached by their 64-bit address in global memory
+// (load_p / store_p), so a thread walks its elements with one address.
+#define RK_GLOBAL(T, p) reinterpret_cast<T __attribute__((address_space(1)))*>(p)
+template <class IO, class = void> struct HasPtr { static constexpr bool value = false; };
+template <class IO> struct HasPtr<IO, decltype((void)IO::kPtr)> { static constexpr bool value = true; };
+
 template <bool NTL, bool NTS = NTL, class X = float2> struct GlobalIO {
     using value_type = X;
     static constexpr bool kBranchFree = true;
+    static constexpr bool kPtr = true;
     __device__ __forceinline__ X load(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*m*/, rk_u64 /*i*/,
                                       rk_i64 addr) const {
-        const X* p = reinterpret_cast<const X*>(a.in) + addr;
-        if constexpr (NTL) {
-            const rk_v2<real_t<X>> x = __builtin_nontemporal_load(reinterpret_cast<const rk_v2<real_t<X>>*>(p));
-            return cx<X>(x.x, x.y);
-        } else {
-            return *p;
-        }
+        return load_p(reinterpret_cast<rk_u64>(reinterpret_cast<const X*>(a.in) + addr));
+    }
+    __device__ __forceinline__ X load_p(rk_u64 p) const {
+        auto q = RK_GLOBAL(const rk_v2<real_t<X>>, p);
+        rk_v2<real_t<X>> x;
+        if constexpr (NTL) x = __builtin_nontemporal_load(q);
+        else x = *q;
+        return cx<X>(x.x, x.y);
     }
     __device__ __forceinline__ void store(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*k*/, rk_u64 /*i*/,
                                           rk_i64 addr, X v) const {
-        X* p = reinterpret_cast<X*>(a.out) + addr;
-        if constexpr (NTS) {
-            rk_v2<real_t<X>> x;
-            x.x = v.x;
-            x.y = v.y;
-            __builtin_nontemporal_store(x, reinterpret_cast<rk_v2<real_t<X>>*>(p));
-        } else {
-            *p = v;
-        }
+        store_p(reinterpret_cast<rk_u64>(reinterpret_cast<X*>(a.out) + addr), v);
+    }
+    __device__ __forceinline__ void store_p(rk_u64 p, X v) const {
+        auto q = RK_GLOBAL(rk_v2<real_t<X>>, p);
+        const rk_v2<real_t<X>> x = {v.x, v.y};
+        if constexpr (NTS) __builtin_nontemporal_store(x, q);
+        else *q = x;
     }
 };
 using PlainIO = GlobalIO<false>;
@@ -599,31 +591,22 @@ typedef float rk_v4u __attribute__((ext_vector_type(4), aligned(8)));
 template <bool NTL, bool NTS = NTL> struct PairIO {
     using value_type = cpair2;
     static constexpr bool kBranchFree = true;
-    __device__ __forceinline__ cpair2 load(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*m*/, rk_u64 /*i*/,
-                                           rk_i64 addr) const {
-        const rk_v4u* p = reinterpret_cast<const rk_v4u*>(a.in + addr);
+    static constexpr bool kPtr = true;
+    __device__ __forceinline__ cpair2 load_p(rk_u64 p) const {
+        auto q = RK_GLOBAL(const rk_v4u, p);
         rk_v4u v;
-        if constexpr (NTL) v = __builtin_nontemporal_load(p);
-        else v = *p;
+        if constexpr (NTL) v = __builtin_nontemporal_load(q);
+        else v = *q;
         return cx<cpair2>(rk_v2<float>{v.x, v.z}, rk_v2<float>{v.y, v.w});
     }
-    // one instance's element (padded sides, where a pair may straddle the edge)
-    __device__ __forceinline__ float2 load_one(const rk_pass_args& a, rk_i64 addr) const { return a.in[addr]; }
-    // two consecutive complex values at addr
-    __device__ __forceinline__ void store_run(const rk_pass_args& a, rk_i64 addr, float x0, float y0, float x1,
-                                              float y1) const {
-        rk_v4u* p = reinterpret_cast<rk_v4u*>(a.out + addr);
+    // two consecutive complex values at p
+    __device__ __forceinline__ void store_run(rk_u64 p, float x0, float y0, float x1, float y1) const {
+        auto q = RK_GLOBAL(rk_v4u, p);
         const rk_v4u v = {x0, y0, x1, y1};
-        if constexpr (NTS) __builtin_nontemporal_store(v, p);
-        else *p = v;
+        if constexpr (NTS) __builtin_nontemporal_store(v, q);
+        else *q = v;
     }
-    __device__ __forceinline__ void store(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*k*/, rk_u64 /*i*/, rk_i64 addr,
-                                          cpair2 v) const {
-        store_run(a, addr, v.x.x, v.y.x, v.x.y, v.y.y);
-    }
-    __device__ __forceinline__ void store_one(const rk_pass_args& a, rk_i64 addr, float x, float y) const {
-        a.out[addr] = make_float2(x, y);
-    }
+    __device__ __forceinline__ void store_p(rk_u64 p, cpair2 v) const { store_run(p, v.x.x, v.y.x, v.x.y, v.y.y); }
 };
 
 // Plain strided IO whose loads and stores are coherent across the whole
@@ -637,16 +620,22 @@ template <bool NTL, bool NTS = NTL> struct PairIO {
 struct CoherentIO {
     using value_type = float2;
     static constexpr bool kBranchFree = true;
+    static constexpr bool kPtr = true;
     __device__ __forceinline__ float2 load(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*m*/, rk_u64 /*i*/,
                                            rk_i64 addr) const {
-        const rk_u64 bits = __hip_atomic_load(reinterpret_cast<rk_u64*>(const_cast<float2*>(a.in + addr)),
-                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return load_p(reinterpret_cast<rk_u64>(a.in + addr));
+    }
+    __device__ __forceinline__ float2 load_p(rk_u64 p) const {
+        const rk_u64 bits = __hip_atomic_load(RK_GLOBAL(rk_u64, p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return make_float2(__uint_as_float((unsigned)bits), __uint_as_float((unsigned)(bits >> 32)));
     }
     __device__ __forceinline__ void store(const rk_pass_args& a, rk_u64 /*o*/, rk_u64 /*k*/, rk_u64 /*i*/,
                                           rk_i64 addr, float2 v) const {
+        store_p(reinterpret_cast<rk_u64>(a.out + addr), v);
+    }
+    __device__ __forceinline__ void store_p(rk_u64 p, float2 v) const {
         const rk_u64 bits = (rk_u64)__float_as_uint(v.x) | ((rk_u64)__float_as_uint(v.y) << 32);
-        __hip_atomic_store(reinterpret_cast<rk_u64*>(a.out + addr), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(RK_GLOBAL(rk_u64, p), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 };
 
@@ -724,9 +713,8 @@ template <int V> __host__ __device__ constexpr bool lower_in(int R) { return pad
 template <int V> __host__ __device__ constexpr bool lower_out(int R) { return pad_out<V>() && R % 2 == 0; }
 
 // One thread's walk over the positions p0 + c of one instance on one side
-// (c a compile-time offset): axis position and element address advance by
-// uniform steps computed once per thread, so an element costs one add and no
-// multiply.
+// (c a compile-time offset): axis position and element address of position p0
+// and their uniform steps per unit of c, formed once per thread.
 struct Walk {
     rk_u64 m0, mstep;   // axis position of position p0, and per unit of c
     rk_i64 a0, astep;   // element address of position p0, and per unit of c
@@ -751,105 +739,170 @@ __device__ __forceinline__ Walk out_walk(const rk_pass_args& a, const Inst& ic, 
     return w;
 }
 
-// Loads position p0 + c of the walk's instance (raw: no sign, no pre-op).  An
-// invalid instance (past n_inst) was decomposed as instance 0, so its
-// addresses are valid: it reads them and its results are never stored.
-template <int V, class IO>
-__device__ __forceinline__ typename IO::value_type load_at(const rk_pass_args& a, const IO& io, const Inst& ic,
-                                                           const Walk& w, int c) {
-    using X = typename IO::value_type;
-    const rk_u64 m = w.m0 + (rk_u64)c * w.mstep;
-    const rk_i64 addr = w.a0 + (rk_i64)c * w.astep;
-    const X zero = cx<X>((real_t<X>)0, (real_t<X>)0);
-    if constexpr (pad_in<V>() && pair_width<X>() == 2) {
-        // the pair may straddle the edge of the data: one load per instance,
-        // each at its own address or its instance's first position
-        const rk_u64 st = pair_step(a);
-        const rk_i64 next = ic.in_base + (rk_i64)(m + st) * a.in_sa + (st ? 0 : a.in_si);
-        const bool ok0 = ic.valid && m < a.n_valid_in, ok1 = ic.valid && m + st < a.n_valid_in;
-        const rk_u64 spare_m = ic.jpass < a.n_valid_in ? ic.jpass : 0;
-        const rk_i64 spare = ic.in_base + (rk_i64)spare_m * a.in_sa;
-        const float2 v0 = io.load_one(a, ok0 ? addr : spare), v1 = io.load_one(a, ok1 ? next : spare);
-        return cx<X>(rk_v2<float>{ok0 ? v0.x : 0.0f, ok1 ? v1.x : 0.0f}, rk_v2<float>{ok0 ? v0.y : 0.0f, ok1 ? v1.y : 0.0f});
-    } else if constexpr (pad_in<V>()) {
-        const bool ok = ic.valid && m < a.n_valid_in;
-        if constexpr (IO::kBranchFree) {
-            // a lane with nothing to load reads its instance's first position
-            // (a valid address, different per instance) and discards it: one
-            // shared clamp address would be a hot spot for loads that bypass
-            // the caches
-            const rk_u64 spare_m = ic.jpass < a.n_valid_in ? ic.jpass : 0;
-            const rk_i64 spare = ic.in_base + (rk_i64)spare_m * a.in_sa;
-            const X y = io.load(a, ic.o, ok ? m : spare_m, ic.i, ok ? addr : spare);
-            return c_select(ok, y, zero);
-        } else {
-            return ok ? io.load(a, ic.o, m, ic.i, addr) : zero;
-        }
-    } else {
-        if constexpr (IO::kBranchFree) {
-            return io.load(a, ic.o, m, ic.i, addr);
-        } else {
-            return ic.valid ? io.load(a, ic.o, m, ic.i, addr) : zero;
-        }
-    }
+// Address or offset + step, hidden from the optimiser: an element then costs
+// one 64-bit add.  Left alone, the compiler rewrites a thread's unrolled
+// addresses p0 + r * step into one or two quarter-rate 64-bit multiply-adds and
+// register moves per element, a quarter of the 256-point column tile's VALU
+// cycles; the same for the stage-twiddle offsets.  walk_step is the uniform
+// byte step, kept in scalar registers.  With the direction's conjugation and
+// scale behind a branch instead of selects: 33 x 65521 87 -> 74 us, 4096 x 997
+// 38.8 -> 35.2, 64 x 2^20 393 -> 375, 1 x 2^20 28.7 -> 26.8.
+__device__ __forceinline__ rk_i64 walk_step(rk_i64 step) {
+    asm("" : "+s"(step));
+    return step;
+}
+__device__ __forceinline__ rk_u64 step_addr(rk_u64 p, rk_i64 step) {
+    p += (rk_u64)step;
+    asm("" : "+v"(p));
+    return p;
+}
+__device__ __forceinline__ rk_u32 step_off(rk_u32 off, rk_u32 step) {
+    off += step;
+    asm("" : "+v"(off));
+    return off;
 }
 
-// Input-side pre-processing of n loaded values at positions p0 + c_i
-// (c_i = cpos(i)): conjugation for the inverse direction (a uniform branch),
-// then the Bluestein chirp (compile-time).  The inter-pass twiddle (PRE_TWIDDLE)
-// is applied by the caller's TwiddleWalk.
-template <int V, int NV, class X, class FC>
-__device__ __forceinline__ void pre_ops(const rk_pass_args& a, const Inst& ic, const Walk& w, X* x, FC cpos) {
-    if (a.in_sign < 0.0f) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) x[i].y = -x[i].y;
-    }
-    if constexpr (Variant<V>::PRE == RK_VAR_PRE_CHIRP) {
+// Loads the values x[i] at positions p0 + i*CS of the walk's instance (raw: no
+// sign, no pre-op).  An invalid instance (past n_inst) was decomposed as
+// instance 0, so its addresses are valid: it reads them and its results are
+// never stored.  On a padded side a lane with nothing to load reads its
+// instance's first position (a valid address, different per instance: one
+// shared clamp address would be a hot spot for loads that bypass the caches),
+// which the zeros behind the chirp table's end turn into zero; N > M/4 (M is
+// the smallest length the planner takes), so positions of the first quarter
+// need no bound (NQ values).
+template <int V, int NV, int CS, int NQ, class IO>
+__device__ __forceinline__ void load_run(const rk_pass_args& a, const IO& io, const Inst& ic, const Walk& w,
+                                         typename IO::value_type* x) {
+    using X = typename IO::value_type;
+    constexpr bool PAD = pad_in<V>();
+    const rk_u64 spare_m = PAD && ic.jpass >= a.n_valid_in ? 0 : ic.jpass;
+    const rk_i64 spare = ic.in_base + (rk_i64)spare_m * a.in_sa;
+    if constexpr (HasPtr<IO>::value) {
+        rk_u64 p = reinterpret_cast<rk_u64>(table<X>(a.in) + w.a0);
+        const rk_u64 sp = reinterpret_cast<rk_u64>(table<X>(a.in) + spare);
+        const rk_i64 st = walk_step(CS * w.astep * (rk_i64)sizeof(scalar_t<X>));
+        rk_u64 m = w.m0;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const rk_u64 m = w.m0 + (rk_u64)cpos(i) * w.mstep;
-            const bool ok = ic.valid && m < a.n_valid_in;
-            const rk_u64 m2 = m + pair_step(a);
-            x[i] = c_mul(x[i], table_at<X>(a.chirp, ok ? m : 0, m2 < a.n_valid_in ? m2 : 0));
+            if (PAD && i >= NQ) x[i] = io.load_p(m < a.n_valid_in ? p : sp);
+            else x[i] = io.load_p(p);
+            if (i + 1 < NV) p = step_addr(p, st);
+            m += (rk_u64)CS * w.mstep;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const rk_u64 m = w.m0 + (rk_u64)(i * CS) * w.mstep;
+            const rk_i64 addr = w.a0 + (rk_i64)(i * CS) * w.astep;
+            const bool ok = ic.valid && (!PAD || m < a.n_valid_in);
+            if constexpr (IO::kBranchFree && PAD)
+                x[i] = io.load(a, ic.o, m < a.n_valid_in ? m : spare_m, ic.i, m < a.n_valid_in ? addr : spare);
+            else if constexpr (IO::kBranchFree)
+                x[i] = io.load(a, ic.o, m, ic.i, addr);
+            else
+                x[i] = ok ? io.load(a, ic.o, m, ic.i, addr) : cx<X>((real_t<X>)0, (real_t<X>)0);
         }
     }
 }
 
-// The output-side operations of one value at axis position kabs: the
-// compile-time post-op, then conjugation and scale for the direction.
+// Input-side pre-processing of the values of load_run: conjugation for the
+// inverse direction (first passes only, which have no inter-pass twiddle; the
+// empty asm keeps the uniform branch a branch instead of selects per value),
+// then the Bluestein chirp (compile-time).  The inter-pass twiddle
+// (PRE_TWIDDLE) is applied by the caller's TwiddleWalk.
+template <int V, int NV, int CS, class X>
+__device__ __forceinline__ void pre_ops(const rk_pass_args& a, const Walk& w, X* x) {
+    if constexpr (Variant<V>::PRE != RK_VAR_PRE_TWIDDLE) {
+        if (a.in_sign < 0.0f) {
+            asm volatile("");
+#pragma unroll
+            for (int i = 0; i < NV; ++i) x[i].y = -x[i].y;
+        }
+    }
+    if constexpr (Variant<V>::PRE == RK_VAR_PRE_CHIRP) {
+        rk_u64 p = reinterpret_cast<rk_u64>(table<X>(a.chirp) + w.m0);
+        const rk_i64 st = walk_step(CS * (rk_i64)w.mstep * (rk_i64)sizeof(scalar_t<X>));
+        const GlobalIO<false, false, scalar_t<X>> tab;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            x[i] = c_mul(x[i], tab.load_p(p));
+            if (i + 1 < NV) p = step_addr(p, st);
+        }
+    }
+}
+
+// The direction's conjugation and scale of an output value.
 template <class X> __device__ __forceinline__ X adjust_out(const rk_pass_args& a, X y) {
     y.y *= (real_t<X>)a.out_sign;
     return c_scale(y, out_scale_of<X>(a));
 }
-
-template <int V, class X>
-__device__ __forceinline__ X post_op(const rk_pass_args& a, rk_u64 kabs, rk_u64 kabs2, X y, bool adjust) {
-    constexpr int POST = Variant<V>::POST;
-    if constexpr (POST == RK_VAR_POST_KMUL_CONJ) y = c_conj(c_mul(y, table_at<X>(a.bspec, kabs, kabs2)));
-    if constexpr (POST == RK_VAR_POST_CONJ_CHIRP) y = c_mul(c_conj(y), table_at<X>(a.chirp, kabs, kabs2));
-    if (adjust) y = adjust_out(a, y);
-    return y;
+template <int N, class X> __device__ __forceinline__ void adjust_all(const rk_pass_args& a, X* y, bool adjust) {
+    if (adjust) {
+        asm volatile("");   // a branch, not selects per value
+#pragma unroll
+        for (int i = 0; i < N; ++i) y[i] = adjust_out(a, y[i]);
+    }
 }
 
-// Stores position k0 + c of the walk's instance (the caller skips invalid
-// instances); a padded side skips positions at or beyond n_valid_out.
-template <int V, class IO>
-__device__ __forceinline__ void store_at(const rk_pass_args& a, const IO& io, const Inst& ic, const Walk& w, int c,
-                                         typename IO::value_type y, bool adjust) {
+// Stores the values y[q*RS + r] at positions k0 + q*SQ + r*SR of the walk's
+// instance (q < NQ, r < NR; the caller skips invalid instances): the
+// compile-time post-op, the direction's adjustment, the store.  valid(q)
+// excludes a thread's idle butterflies; a padded side skips positions at or
+// beyond n_valid_out (those of its first quarter never are: NU values of r).
+template <int V, int NQ, int SQ, int NR, int SR, int RS, int NU, class IO, class FV>
+__device__ __forceinline__ void store_run(const rk_pass_args& a, const IO& io, const Inst& ic, const Walk& w,
+                                          typename IO::value_type* y, bool adjust, FV valid) {
     using X = typename IO::value_type;
-    const rk_u64 kabs = w.m0 + (rk_u64)c * w.mstep;
-    if constexpr (pad_out<V>())
-        if (kabs >= a.n_valid_out) return;
-    // a DIRECT store's pair is adjacent along I, or along NS (position + 1)
-    const rk_u64 k2 = kabs + (pair_width<X>() == 2 ? pair_step(a) : 0);
-    const rk_i64 addr = w.a0 + (rk_i64)c * w.astep;
-    if constexpr (pad_out<V>() && pair_width<X>() == 2) {
-        const bool two = k2 < a.n_valid_out;
-        y = post_op<V>(a, kabs, two ? k2 : kabs, y, adjust);
-        if (two) io.store(a, ic.o, kabs, ic.i, addr, y);
-        else io.store_one(a, addr, y.x.x, y.y.x);
+    constexpr int POST = Variant<V>::POST;
+    if constexpr (POST != RK_VAR_POST_NONE) {
+        const rk_i64 es = (rk_i64)sizeof(scalar_t<X>);
+        const rk_i64 sr = walk_step(SR * (rk_i64)w.mstep * es), sq = walk_step(SQ * (rk_i64)w.mstep * es);
+        rk_u64 pr = reinterpret_cast<rk_u64>(table<X>(POST == RK_VAR_POST_KMUL_CONJ ? a.bspec : a.chirp) + w.m0);
+        const GlobalIO<false, false, scalar_t<X>> tab;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            rk_u64 p = pr;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                X& v = y[q * RS + r];
+                if (valid(q)) {
+                    if constexpr (POST == RK_VAR_POST_KMUL_CONJ) v = c_conj(c_mul(v, tab.load_p(p)));
+                    else v = c_mul(c_conj(v), tab.load_p(p));
+                }
+                if (q + 1 < NQ) p = step_addr(p, sq);
+            }
+            if (r + 1 < NR) pr = step_addr(pr, sr);
+        }
+    }
+    adjust_all<(NQ - 1) * RS + NR>(a, y, adjust);
+    const rk_u64 k00 = w.m0;
+    if constexpr (HasPtr<IO>::value) {
+        const rk_i64 es = (rk_i64)sizeof(scalar_t<X>);
+        const rk_i64 sr = walk_step(SR * w.astep * es), sq = walk_step(SQ * w.astep * es);
+        rk_u64 pr = reinterpret_cast<rk_u64>(table<X>(a.out) + w.a0);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            rk_u64 p = pr;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const bool ok = !pad_out<V>() || r < NU || k00 + (rk_u64)(q * SQ + r * SR) * w.mstep < a.n_valid_out;
+                if (valid(q) && ok) io.store_p(p, y[q * RS + r]);
+                if (q + 1 < NQ) p = step_addr(p, sq);
+            }
+            if (r + 1 < NR) pr = step_addr(pr, sr);
+        }
     } else {
-        io.store(a, ic.o, kabs, ic.i, addr, post_op<V>(a, kabs, k2, y, adjust));
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const int c = q * SQ + r * SR;
+                const rk_u64 kabs = k00 + (rk_u64)c * w.mstep;
+                const bool ok = !pad_out<V>() || kabs < a.n_valid_out;
+                if (valid(q) && ok) io.store(a, ic.o, kabs, ic.i, w.a0 + (rk_i64)c * w.astep, y[q * RS + r]);
+            }
+        }
     }
 }
 
@@ -879,12 +932,14 @@ template <bool WAVE> __device__ __forceinline__ void exchange_sync() {
     }
 }
 
-template <bool SPLIT, int NW, int NR, bool WAVE = false, class X, class FW, class FR>
+// LEAD: LDS may still be read from an earlier exchange, so the writes wait for
+// every thread (not needed by a tile's first exchange).
+template <bool SPLIT, int NW, int NR, bool WAVE = false, bool LEAD = true, class X, class FW, class FR>
 __device__ __forceinline__ void lds_exchange(void* base, const X* w, X* r, FW wpos, FR rpos) {
     using F = real_t<X>;
     if constexpr (!SPLIT) {
         X* lds = reinterpret_cast<X*>(base);
-        exchange_sync<WAVE>();
+        if constexpr (LEAD) exchange_sync<WAVE>();
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
             const int p = wpos(i);
@@ -901,7 +956,7 @@ __device__ __forceinline__ void lds_exchange(void* base, const X* w, X* r, FW wp
         F wy[NW], rx[NR];
 #pragma unroll
         for (int i = 0; i < NW; ++i) wy[i] = w[i].y;
-        exchange_sync<WAVE>();
+        if constexpr (LEAD) exchange_sync<WAVE>();
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
             const int p = wpos(i);
@@ -1032,7 +1087,8 @@ RK_HD constexpr int flat_pair_lds(int tid, int it, int b) {
 template <int T> RK_HD constexpr int col_lds(int ps, int it) { return lds_pad_add<(T < 16 ? T : 16)>(ps, it * T); }
 
 // LOWER: the upper half of the first stage's inputs is zero (lower_in).
-template <int L, int S, bool SPLIT, int VM, bool WAVE = false, bool LOWER = false, class X>
+// LEAD0: the first exchange is not the tile's first use of LDS.
+template <int L, int S, bool SPLIT, int VM, bool WAVE = false, bool LOWER = false, bool LEAD0 = true, class X>
 __device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const scalar_t<X>* twl) {
     using P = Plan<L>;
     constexpr int R = P::radix(S);
@@ -1046,9 +1102,15 @@ __device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const sc
             const int j = t + q * T;
             if (stage_valid<L, S>(t, q)) {
                 const int m = j % NS;
+                // byte offset of W_L^{r*m*L/(NS*R)}, one add per r
+                const rk_u32 step = (rk_u32)m * (L / (NS * R)) * (rk_u32)sizeof(scalar_t<X>);
+                rk_u32 off = 0;
 #pragma unroll
-                for (int r = 1; r < R; ++r)
-                    v[q * R + r] = c_mul(v[q * R + r], twl[(r * m) * (L / (NS * R))]);
+                for (int r = 1; r < R; ++r) {
+                    off = step_off(off, step);
+                    v[q * R + r] = c_mul(v[q * R + r], *reinterpret_cast<const scalar_t<X>*>(
+                                                           reinterpret_cast<const char*>(twl) + off));
+                }
             }
         }
     }
@@ -1061,7 +1123,7 @@ __device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const sc
     if constexpr (S + 1 < P::NSTAGE) {
         constexpr int R1 = P::radix(S + 1);
         constexpr int Q1 = P::q(S + 1);
-        lds_exchange<SPLIT, Q * R, Q1 * R1, WAVE>(
+        lds_exchange<SPLIT, Q * R, Q1 * R1, WAVE, (LEAD0 || S > 0)>(
             my, v, v,
             [&](int i) { return stage_valid<L, S>(t, i / R) ? stage_out_lds<L, S>(t, i) : -1; },
             [&](int i) { return stage_valid<L, S + 1>(t, i / R1) ? stage_in_lds<L, S + 1>(t, i) : -1; });
@@ -1073,18 +1135,19 @@ __device__ __forceinline__ void run_stages(X (&v)[VM], void* my, int t, const sc
 // the pass kernel body
 // ------------------------------------------------------------------------
 // Tile of this work-group.  The dispatcher hands work-group b to XCD
-// b % n_xcd; with xcd_group = G > 1 the G tiles of each group of consecutive
+// b % n_xcd; with groups of G > 1 the G tiles of each group of consecutive
 // tiles go to work-groups on one XCD, so tiles that share cache lines (narrow
 // column tiles) share that XCD's L2 instead of each fetching whole lines.
+// Both counts are powers of two: scalar shifts, where four divisions cost
+// about 80 vector instructions per wave.
 __device__ __forceinline__ rk_u64 xcd_tile(const rk_pass_args& a) {
     const rk_u32 b = blockIdx.x;
-    const rk_u32 g = a.xcd_group, nx = a.n_xcd;
-    if (g <= 1) return b;
-    const rk_u32 span = g * nx;
-    const rk_u32 full = (gridDim.x / span) * span;
+    const rk_u32 g = a.xcd_group_lg, nx = a.n_xcd_lg;
+    if (g == 0) return b;
+    const rk_u32 full = (gridDim.x >> (g + nx)) << (g + nx);
     if (b >= full) return b;
-    const rk_u32 x = b % nx, k = b / nx;
-    return (rk_u64)(k / g) * span + x * g + (k % g);
+    const rk_u32 x = b & ((1u << nx) - 1), k = b >> nx;
+    return ((rk_u64)(k >> g) << (g + nx)) + (x << g) + (k & ((1u << g) - 1));
 }
 
 // LDS bytes of a tile and whether its exchanges are split into halves.
@@ -1115,6 +1178,18 @@ template <int L, int C, bool HALF, class X> __host__ __device__ constexpr int ti
     return tile_lds_bytes<L, C, HALF, (int)sizeof(scalar_t<X>)>();
 }
 
+// Instances left from inst0 on, cut to 32 bits (the tile compares them with
+// its C).  The high word goes through an empty asm: of a 64-bit compare whose
+// result both selects and branches, the compiler (ROCm 7.2) dropped the
+// instruction that sets the select's condition, and ragged tiles of short rows
+// were stored whole, past the end of the output.
+__device__ __forceinline__ rk_u32 instances_left(const rk_pass_args& a, rk_u64 inst0) {
+    const rk_u64 left = a.n_inst - inst0;
+    rk_u32 hi = (rk_u32)(left >> 32);
+    asm("" : "+s"(hi));
+    return hi ? 0x7fffffffu : (rk_u32)left;
+}
+
 // One tile (instances tile*C ... tile*C + C - 1) computed by threads
 // tid = 0 ... C*T - 1 with `lds` of at least tile_lds_bytes<L, C, HALF, ES>()
 // bytes (ES = sizeof the IO policy's element type).
@@ -1128,13 +1203,13 @@ template <int L, int C, int V, class IO, int MODES = 0, bool WAVE = false, bool 
           bool TWLDS = false>
 __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& io, typename IO::value_type* lds,
                                               rk_u64 tile, int tid, const typename IO::value_type* pre = nullptr,
-                                              const scalar_t<typename IO::value_type>* twl_lds = nullptr) {
+                                              scalar_t<typename IO::value_type>* twl_lds = nullptr) {
     using X = typename IO::value_type;
     using F = real_t<X>;
     constexpr int W = pair_width<X>();   // instances per thread
     constexpr int CT = C / W;
     static_assert(W == 1 || (C % 2 == 0 && MODES && (MODES & 3) == RK_MODE_DIRECT && !WAVE && !PRE && !HALF &&
-                             !Variant<V>::BLUE && ((MODES >> 2) & 3) != RK_MODE_ROW),
+                             !Variant<V>::BLUE && !pad_in<V>() && Variant<V>::POST == RK_VAR_POST_NONE && ((MODES >> 2) & 3) != RK_MODE_ROW),
                   "pairs of instances: column tiles with DIRECT loads and DIRECT or FLAT stores");
     using P = Plan<L>;
     static_assert(!WAVE || (64 % P::T == 0), "wave-local stages need whole instances per wave");
@@ -1168,6 +1243,30 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     X v[VM];
     X g[R0];   // staging registers (global side of a staged load/store)
 
+    // With TWLDS the tile copies the stage twiddles W_L^e into twl_lds.  Their
+    // loads are issued before the tile's own and written to LDS once those are
+    // on their way too (the first exchange's barrier publishes them), so the
+    // tile waits for memory once, not twice; the scheduling barrier keeps the
+    // first use of a loaded value behind the last load.  A tile that is one
+    // round of latencies shows it most: with both, 4096 x 1000 16.9 -> 15.4
+    // us, 2048 x 2048 16.9 -> 14.7, 16384 x 256 13.0 -> 11.9, 4096 x 997 35.2
+    // -> 32.3, 8192 x 1024 29.7 -> 27.9.
+    constexpr int NTW = TWLDS ? (L + NT - 1) / NT : 1;
+    scalar_t<X> tw[NTW];
+    if constexpr (TWLDS) {
+        const scalar_t<X>* tab = table<X>(a.twl);
+#pragma unroll
+        for (int k = 0; k < NTW; ++k) tw[k] = tab[L % NT == 0 || tid + k * NT < L ? tid + k * NT : 0];
+    }
+    auto loads_issued = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (TWLDS) {
+#pragma unroll
+            for (int k = 0; k < NTW; ++k)
+                if (L % NT == 0 || tid + k * NT < L) twl_lds[tid + k * NT] = tw[k];
+        }
+    };
+
     // ---- stage-0 inputs: element p = t + r*T of instance c ----
     const Inst ic = decompose<L>(a, inst0 + c * W);
     auto own_pos = [&](int i) { return cbase + stage_in_lds<L, 0>(t, i); };
@@ -1177,47 +1276,52 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
 #pragma unroll
             for (int r = 0; r < NL; ++r) v[r] = pre[r];
         } else {
-#pragma unroll
-            for (int r = 0; r < NL; ++r) v[r] = load_at<V, IO>(a, io, ic, w, r * T);
+            load_run<V, NL, T, R0 / 4>(a, io, ic, w, v);
         }
-        pre_ops<V, NL>(a, ic, w, v, [](int r) { return r * T; });
+        loads_issued();
+        pre_ops<V, NL, T>(a, w, v);
         if constexpr (TWID) apply_pass_twiddles<R0>(a, ic.l, t, T, v);
     } else if constexpr (W == 2) {
         // pairs load DIRECT
     } else if (load_mode == RK_MODE_FLAT) {
         // instance-linear block of C*L elements, no pre-ops
         const rk_i64 base = a.in_off + (rk_i64)inst0 * L;
+        const rk_u32 left = instances_left(a, inst0);
 #pragma unroll
         for (int it = 0; it < R0; ++it) {
             const int e = tid + it * NT;
             const int ce = e / L, p = e - ce * L;
-            X x = cx<X>((F)0, (F)0);
-            const bool ok = inst0 + ce < a.n_inst;
-            if constexpr (IO::kBranchFree) {
-                // a lane past the last instance loads the tile's first element
-                const X y = io.load(a, ok ? inst0 + ce : inst0, ok ? p : 0, 0, ok ? base + e : base);
-                x = c_select(ok, y, x);
+            // a lane past the last instance loads the tile's first element; its
+            // results are never stored
+            const bool ok = (rk_u32)ce < left;
+            if constexpr (HasPtr<IO>::value) {
+                const rk_u64 at = reinterpret_cast<rk_u64>(table<X>(a.in) + base);
+                g[it] = io.load_p(at + (ok ? (rk_u32)e * (rk_u32)sizeof(X) : 0u));
+            } else if constexpr (IO::kBranchFree) {
+                g[it] = io.load(a, ok ? inst0 + ce : inst0, ok ? p : 0, 0, ok ? base + e : base);
             } else {
-                if (ok) x = io.load(a, inst0 + ce, p, 0, base + e);
+                g[it] = cx<X>((F)0, (F)0);
+                if (ok) g[it] = io.load(a, inst0 + ce, p, 0, base + e);
             }
-            g[it] = x;
         }
+        loads_issued();
         if (a.in_sign < 0.0f) {
+            asm volatile("");
 #pragma unroll
             for (int it = 0; it < R0; ++it) g[it].y = -g[it].y;
         }
-        lds_exchange<SPLIT, R0, R0>(
+        lds_exchange<SPLIT, R0, R0, false, PRE>(
             lds, g, v,
             [&](int it) { return flat_lds<L, NT, LP>(tid, it); }, own_pos);
     } else {
         // COLUMN (under the row mapping) or ROW (under the column mapping)
         const Inst ics = decompose<L>(a, inst0 + cs);
         const Walk w = in_walk(a, ics, ps);
-#pragma unroll
-        for (int it = 0; it < NL; ++it) g[it] = load_at<V, IO>(a, io, ics, w, it * T);
-        pre_ops<V, NL>(a, ics, w, g, [](int it) { return it * T; });
+        load_run<V, NL, T, R0 / 4>(a, io, ics, w, g);
+        loads_issued();
+        pre_ops<V, NL, T>(a, w, g);
         if constexpr (TWID) apply_pass_twiddles<R0>(a, ics.l, ps, T, g);
-        lds_exchange<SPLIT, NL, NL>(
+        lds_exchange<SPLIT, NL, NL, false, PRE>(
             lds, g, v, [&](int it) { return cs * LP + col_lds<T>(ps, it); }, own_pos);
     }
 
@@ -1229,7 +1333,8 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     const scalar_t<X>* twl;
     if constexpr (TWLDS) twl = twl_lds;
     else twl = table<X>(a.twl);
-    run_stages<L, 0, SPLIT, VM, WAVE, LOW>(v, my, t, twl);
+    constexpr bool LEAD0 = PRE || !(MODES && (MODES & 3) == RK_MODE_DIRECT);
+    run_stages<L, 0, SPLIT, VM, WAVE, LOW, LEAD0>(v, my, t, twl);
 
     if constexpr (BLUE) {
         // A = FFT(chirp * x): multiply by the kernel spectrum, conjugate, and
@@ -1237,8 +1342,8 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
 #pragma unroll
         for (int i = 0; i < QL * RL; ++i)
             if (stage_valid<L, SL>(t, i / RL)) {
-                const int k = stage_out_pos<L, SL>(t, i);
-                v[i] = c_conj(c_mul(v[i], table<X>(a.bspec)[k]));
+                // position t + (q*T + r*NS): a constant offset from one address
+                v[i] = c_conj(c_mul(v[i], (table<X>(a.bspec) + t)[stage_out_pos<L, SL>(0, i)]));
             }
         lds_exchange<SPLIT, QL * RL, R0, WAVE>(lds, v, v, last_out, own_pos);
         // the second transform and the stores recompute what depends on the
@@ -1254,73 +1359,67 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     // ---- store: output element k = stage_out_pos of the last stage ----
     const bool adjust = a.out_sign < 0.0f || a.out_scale != 1.0f;
     if (store_mode == RK_MODE_DIRECT) {
-        // last stage: butterfly j = t + q*T < NS, so output k = t + stage_out_pos(0, i)
+        // last stage: butterfly j = t + q*T < NS
         static_assert(P::nb(SL) == P::ns(SL), "the last Stockham stage writes its outputs at j + r * NS");
         if (ic.valid) {
-            const Walk w = out_walk(a, ic, t);
-#pragma unroll
-            for (int i = 0; i < QL * RL; ++i)
-                if (!(lower_out<V>(RL) && i % RL >= RL / 2) && stage_valid<L, SL>(t, i / RL)) store_at<V, IO>(a, io, ic, w, stage_out_pos<L, SL>(0, i), v[i], adjust);
+            // last stage: output k = t + q*T + r*NS
+            constexpr int NR = lower_out<V>(RL) ? RL / 2 : RL;
+            store_run<V, QL, T, NR, P::ns(SL), RL, RL / 4>(a, io, ic, out_walk(a, ic, t), v, adjust,
+                                                           [&](int q) { return stage_valid<L, SL>(t, q); });
         }
     } else if constexpr (W == 2) {
         // FLAT: the tile is C*L contiguous elements; a thread takes two
-        // consecutive positions of both instances of a pair where it can
+        // consecutive positions of both instances of a pair (even R0 and L)
+        static_assert(R0 % 2 == 0 && L % 2 == 0, "a pair tile stores two positions at a time");
         const rk_i64 base = a.out_off + (rk_i64)inst0 * L;
-        if constexpr (R0 % 2 == 0 && L % 2 == 0) {
-            lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out,
-                                             [&](int i) { return flat_pair_lds<L, NT, LP>(tid, i / 2, i % 2); });
+        const rk_u32 left = instances_left(a, inst0);
+        lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out,
+                                         [&](int i) { return flat_pair_lds<L, NT, LP>(tid, i / 2, i % 2); });
+        adjust_all<R0>(a, g, adjust);
+        auto store_all = [&](auto keep) {
 #pragma unroll
             for (int it = 0; it < R0 / 2; ++it) {
                 const int e = 2 * (tid + it * NT);
                 const int ce = e / L, k = e - ce * L;
-                if (inst0 + 2 * ce < a.n_inst) {
-                    X y0 = g[2 * it], y1 = g[2 * it + 1];
-                    if (adjust) {
-                        y0 = adjust_out(a, y0);
-                        y1 = adjust_out(a, y1);
-                    }
-                    const rk_i64 at = base + (rk_i64)(2 * ce) * L + k;
-                    io.store_run(a, at, y0.x.x, y0.y.x, y1.x.x, y1.y.x);
-                    io.store_run(a, at + L, y0.x.y, y0.y.y, y1.x.y, y1.y.y);
+                if (keep(2 * ce)) {
+                    const X y0 = g[2 * it], y1 = g[2 * it + 1];
+                    const rk_u64 at = reinterpret_cast<rk_u64>(a.out + base) + (rk_u32)(2 * ce * L + k) * 8u;
+                    io.store_run(at, y0.x.x, y0.y.x, y1.x.x, y1.y.x);
+                    io.store_run(at + L * 8, y0.x.y, y0.y.y, y1.x.y, y1.y.y);
                 }
             }
-        } else {
-            lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return flat_lds<L, NT, LP>(tid, it); });
+        };
+        if (left >= (rk_u32)C) store_all([](int) { return true; });
+        else store_all([&](int ce) { return (rk_u32)ce < left; });
+    } else if (store_mode == RK_MODE_FLAT) {
+        // no post-ops beyond sign and scale
+        lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return flat_lds<L, NT, LP>(tid, it); });
+        adjust_all<R0>(a, g, adjust);
+        const rk_i64 base = a.out_off + (rk_i64)inst0 * L;
+        const rk_u32 left = instances_left(a, inst0);
+        auto store_all = [&](auto keep) {
 #pragma unroll
             for (int it = 0; it < R0; ++it) {
                 const int e = tid + it * NT;
                 const int ce = e / L, k = e - ce * L;
-                if (inst0 + 2 * ce < a.n_inst) {
-                    X y = g[it];
-                    if (adjust) y = adjust_out(a, y);
-                    const rk_i64 at = base + (rk_i64)(2 * ce) * L + k;
-                    io.store_one(a, at, y.x.x, y.y.x);
-                    io.store_one(a, at + L, y.x.y, y.y.y);
+                if (keep(ce)) {
+                    if constexpr (HasPtr<IO>::value)
+                        io.store_p(reinterpret_cast<rk_u64>(table<X>(a.out) + base) + (rk_u32)e * (rk_u32)sizeof(X),
+                                   g[it]);
+                    else
+                        io.store(a, inst0 + ce, k, 0, base + e, g[it]);
                 }
             }
-        }
-    } else if (store_mode == RK_MODE_FLAT) {
-        // no post-ops beyond sign and scale
-        lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return flat_lds<L, NT, LP>(tid, it); });
-        const rk_i64 base = a.out_off + (rk_i64)inst0 * L;
-#pragma unroll
-        for (int it = 0; it < R0; ++it) {
-            const int e = tid + it * NT;
-            const int ce = e / L, k = e - ce * L;
-            if (inst0 + ce < a.n_inst) {
-                X y = g[it];
-                if (adjust) y = adjust_out(a, y);
-                io.store(a, inst0 + ce, k, 0, base + e, y);
-            }
-        }
+        };
+        // one uniform branch, not one per value
+        if (left >= (rk_u32)C) store_all([](int) { return true; });
+        else store_all([&](int ce) { return (rk_u32)ce < left; });
     } else {
         constexpr int NO = lower_out<V>(R0) ? R0 / 2 : R0;
         lds_exchange<SPLIT, QL * RL, NO>(lds, v, g, last_out, [&](int it) { return cs * LP + col_lds<T>(ps, it); });
         const Inst ics = decompose<L>(a, inst0 + cs);
         if (ics.valid) {
-            const Walk w = out_walk(a, ics, ps);
-#pragma unroll
-            for (int it = 0; it < NO; ++it) store_at<V, IO>(a, io, ics, w, it * T, g[it], adjust);
+            store_run<V, 1, 0, NO, T, R0, R0 / 4>(a, io, ics, out_walk(a, ics, ps), g, adjust, [](int) { return true; });
         }
     }
 }
@@ -1362,10 +1461,7 @@ __device__ __forceinline__ void fft_pass_body(const rk_pass_args& a, const IO& i
     const rk_u64 tile = xcd_tile(a) + a.tile_base;
     if (tile >= a.n_tiles) return;
     if constexpr (twl_in_lds<L, C, V, WAVE, HALF, X>()) {
-        // the stage twiddles W_L^e from LDS, published by the tile's first
-        // exchange barrier (before stage 1 reads them)
         __shared__ scalar_t<X> twl_s[L];
-        for (int e = (int)threadIdx.x; e < L; e += CT * Plan<L>::T) twl_s[e] = table<X>(a.twl)[e];
         fft_pass_tile<L, C, V, IO, MODES, WAVE, false, HALF, true>(a, io, lds, tile, (int)threadIdx.x, nullptr, twl_s);
     } else {
         fft_pass_tile<L, C, V, IO, MODES, WAVE, false, HALF>(a, io, lds, tile, (int)threadIdx.x);
@@ -1383,8 +1479,7 @@ __device__ __forceinline__ void direct_raw_loads(const rk_pass_args& a, const IO
     const int t = colmap ? (tid / C) : (tid % T);
     const Inst ic = decompose<L>(a, tile * (rk_u64)C + c);
     const Walk w = in_walk(a, ic, t);
-#pragma unroll
-    for (int r = 0; r < (lower_in<V>(P::R0) ? P::R0 / 2 : P::R0); ++r) raw[r] = load_at<V, IO>(a, io, ic, w, r * T);
+    load_run<V, (lower_in<V>(P::R0) ? P::R0 / 2 : P::R0), T, P::R0 / 4>(a, io, ic, w, raw);
 }
 
 // Persistent, software-pipelined pass (DIRECT loads only): work-group b runs

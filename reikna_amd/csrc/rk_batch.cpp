@@ -306,7 +306,7 @@ void resolve_tables(rk_pass_args& a, const PassPlan& pp, const char* tables) {
     a.chirp = (const float2*)tab(pp.chirp_off);
     a.bspec = (const float2*)tab(pp.bspec_off);
     a.tile_base = 0;
-    a.xcd_group = 0;
+    a.xcd_group_lg = 0;
 }
 
 }  // namespace rk

@@ -68,9 +68,7 @@ __device__ __forceinline__ void run_case(rk_u32 kc, const rk_pass_args& a, float
     case id: {                                                                         \
         constexpr int nt = rkfft::pass_threads<L, C>();                                \
         if constexpr (batch_twl<L, C>()) {                                             \
-            /* published by the tile's first exchange barrier */                        \
             float2* tw = reinterpret_cast<float2*>(reinterpret_cast<char*>(lds) + twl_offset<L, C>()); \
-            for (int e = tid; e < L; e += kThreads) tw[e] = rkfft::table<float2>(a.twl)[e]; \
             rkfft::fft_pass_tile<L, C, V, rkfft::CoherentIO, 0, false, false, false, true>( \
                 a, rkfft::CoherentIO{}, lds, tile, tid < nt ? tid : nt - 1, nullptr, tw); \
         } else {                                                                       \

@@ -598,9 +598,10 @@ int describe_pass(const AxisPass& ap, const Layout& ls, const Layout& ld, int ax
     if ((!(ap.pre_ops & RK_PRE_CHIRP) && ap.n_valid_in != ap.Nax) ||
         (!(ap.post_ops & RK_POST_CHIRP) && ap.n_valid_out != ap.Nax))
         return fail(RK_ERR_UNSUPPORTED, "internal: a padded pass side without a chirp op (L=%d)", ap.L);
-    // ... and skip the upper half of a chirp side's positions (lower_in / lower_out)
-    if (ap.Nax % 2 == 0 && (((ap.pre_ops & RK_PRE_CHIRP) && 2 * ap.n_valid_in > ap.Nax) ||
-                            ((ap.post_ops & RK_POST_CHIRP) && 2 * ap.n_valid_out > ap.Nax)))
+    // ... skip the upper half of a chirp side's positions (lower_in / lower_out)
+    // and bound no position of its first quarter
+    auto fits = [&](int64_t n) { return (ap.Nax % 2 || 2 * n <= ap.Nax) && 4 * n > ap.Nax; };
+    if (((ap.pre_ops & RK_PRE_CHIRP) && !fits(ap.n_valid_in)) || ((ap.post_ops & RK_POST_CHIRP) && !fits(ap.n_valid_out)))
         return fail(RK_ERR_UNSUPPORTED, "internal: Bluestein over %lld points of %lld values", (long long)ap.Nax,
                     (long long)ap.n_valid_in);
     rk_pass_args& a = pp.args;
@@ -702,11 +703,14 @@ static void set_xcd_group(PassPlan& pp) {
         g = (rk_u32)forced;
     else if ((pp.args.cmap || pp.args.load_mode == RK_MODE_COLUMN || pp.args.store_mode == RK_MODE_COLUMN) && C <= 16)
         g = (rk_u32)(32 / C);
-    pp.args.xcd_group = 0;
-    if (g > 1) {
-        pp.args.xcd_group = g;
-        pp.args.n_xcd = xcd_count();
-    }
+    auto log2_floor = [](rk_u32 x) {
+        rk_u32 l = 0;
+        while ((x >>= 1) != 0) ++l;
+        return l;
+    };
+    const rk_u32 n = xcd_count();
+    pp.args.n_xcd_lg = log2_floor(n);
+    pp.args.xcd_group_lg = n & (n - 1) ? 0 : log2_floor(g);
 }
 
 // Bytes above which a plain or twiddle pass uses the streaming kernel: the
@@ -1053,14 +1057,16 @@ int build_tables(TableBuilder& tb, PassPlan& pp, const AxisPass& ap, int64_t nre
     const bool needs_chirp = (ap.pre_ops & RK_PRE_CHIRP) || (ap.post_ops & RK_POST_CHIRP);
     if (needs_chirp) {
         // exp(-i pi (n^2 mod 2N) / N): the phase index is an exact integer
-        std::vector<cd> ch(nreal);
+        // zeros behind its end up to the middle of the axis (the kernels'
+        // upper positions are never loaded): padded inputs times these vanish
+        std::vector<cd> ch(std::max<int64_t>(nreal, ap.Nax), cd(0, 0));
         const int64_t two_n = 2 * nreal;
         for (int64_t k = 0; k < nreal; ++k) {
             const unsigned __int128 sq = (unsigned __int128)k * (unsigned __int128)k;
             const int64_t ph = (int64_t)(sq % (unsigned __int128)two_n);
             ch[k] = unit_root(ph, two_n);   // exp(-2 pi i ph / 2N) = exp(-i pi ph / N)
         }
-        pp.chirp_off = add_table(tb, pp, "chirp" + std::to_string(nreal), ch);
+        pp.chirp_off = add_table(tb, pp, "chirp" + std::to_string(nreal) + "_" + std::to_string(ap.Nax), ch);
     }
     const bool needs_bspec = ap.blue_single || (ap.post_ops & RK_POST_KMUL_CONJ);
     if (needs_bspec) {
@@ -1301,7 +1307,7 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
         set_xcd_group(pp);
         const uint64_t max_grid = (uint64_t(1) << 31) / (uint64_t)pp.threads;
         pp.grid = std::min<uint64_t>(pp.args.n_tiles, pp.pipe ? pipe_grid(pp) : max_grid);
-        if (pp.pipe) pp.args.xcd_group = 1;   // the persistent body walks tiles in launch order
+        if (pp.pipe) pp.args.xcd_group_lg = 0;   // the persistent body walks tiles in launch order
     }
     plan->ws_bytes = 0;
     if (ws_elems) {

@@ -168,11 +168,12 @@ class NativeFftPlan:
 
     def execute(self, out_ptr: int, in_ptr: int, inverse: int, ws_ptr: int | None, stream: int | None,
                 load_blob: bytes | None = None, store_blob: bytes | None = None) -> None:
-        h = ctypes.c_void_p(self.handle)
         if load_blob is None and store_blob is None:
-            rc = _lib.load().rk_fft_execute(h, ctypes.c_void_p(out_ptr), ctypes.c_void_p(in_ptr), int(inverse),
-                                            ctypes.c_void_p(ws_ptr), ctypes.c_void_p(stream))
+            rc = _lib.load().rk_fft_execute(self.handle, out_ptr, in_ptr, inverse, ws_ptr, stream)
+            if rc == _lib.RK_OK:
+                return
         else:
+            h = ctypes.c_void_p(self.handle)
             lb = load_blob or b""
             sb = store_blob or b""
             rc = _lib.load().rk_fft_execute_fused(

@@ -560,6 +560,14 @@ class Array(AsArrayMetadata):
     def size(self) -> int:
         return self.metadata.size
 
+    def matches(self, meta: ArrayMetadata) -> bool:
+        """Whether the array has exactly the layout `meta` in a buffer that holds it."""
+        have = self.metadata
+        size = getattr(self.buffer, "size", None)
+        return (have.shape == meta.shape and have.dtype == meta.dtype and have.strides == meta.strides
+                and have.first_element_offset == meta.first_element_offset
+                and (size is None or size >= meta.buffer_size))
+
     @property
     def ptr(self) -> int:
         """Base pointer of the buffer (element 0 sits at ptr + offset)."""

@@ -253,15 +253,21 @@ def catalog_entries() -> list[tuple[int, int, int]]:
     for length in catalog_lengths():
         if length & (length - 1) and length >= 8 and threads_per_instance(length) < 32:
             ents.add((length, tile_c_row(length), VAR_PLAIN | VAR_MODE_FF))
-    # single-kernel Bluestein tiles up to M = 1024 with DIRECT/DIRECT compiled
-    # in and bounded to three waves per SIMD (at most 168 VGPRs, a few
-    # spilled): 8192 x 251 (M = 512) 24.1 against 28.5 us, 4096 x 509 and
-    # 16384 x 61 4 % faster; from M = 2048 the bound costs more than the
-    # occupancy gives (4096 x 997 69 against 58 us), so those keep the generic
-    # kernel
+    # single-kernel Bluestein tiles with DIRECT/DIRECT compiled in (tiles of at
+    # most 256 threads also bounded to three waves per SIMD): 4096 x 997 (M =
+    # 2048) 32.3 -> 31.0 us, 16 x 2003 11.7 -> 11.5; at M = 8192 the generic
+    # kernel is the faster one (1024 x 4093 71.4 / 72.1)
     for length, c, v in list(ents):
-        if v == VAR_BLUE and length <= 1024 and c * threads_per_instance(length) <= 256:
+        if v == VAR_BLUE and length <= 4096:
             ents.add((length, c, v | VAR_MODE_DD))
+    # the passes of Bluestein chains: 33 x 65521 69.7 -> 68.0 us, 64 x 10007
+    # 44.1 -> 42.5, 200 x 40009 248 -> 242
+    for length, c, v in list(ents):
+        if length <= FACTOR_MAX and c == tile_c_col(length):
+            if v == VAR_CHIRP:
+                ents.add((length, c, v | VAR_MODE_DF))
+            elif v in (VAR_TWIDDLE_KMUL, VAR_TWIDDLE_CONJ_CHIRP):
+                ents.add((length, c, v | VAR_MODE_DD))
     return sorted(ents)
 
 

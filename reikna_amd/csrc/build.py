@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import argparse
 import concurrent.futures
+import functools
 import hashlib
 import os
 import shutil
@@ -42,7 +43,7 @@ N_PARTS = 12
 # ---------------------------------------------------------------------------
 # catalog: mirrors make_radix_list / lds_pitch / tile_c_row / tile_c_col
 # ---------------------------------------------------------------------------
-def radix_list(length: int) -> list[int]:
+def prime_power_list(length: int) -> list[int]:
     x, p2, n3, n5, n7 = length, 0, 0, 0, 0
     while x % 2 == 0:
         x //= 2
@@ -68,6 +69,51 @@ def radix_list(length: int) -> list[int]:
     imax = max(range(len(r)), key=lambda k: (r[k], -k))
     r[0], r[imax] = r[imax], r[0]
     return r
+
+
+# operations of the in-register DFT of each radix (fft_device.hpp make_radix_list)
+RADIX_COST = {16: 168, 15: 200, 12: 112, 10: 100, 9: 120, 8: 60, 7: 84, 6: 40, 5: 40, 4: 16, 3: 16, 2: 4}
+
+
+def _radix_sequences(x: int, limit: int, depth: int = 0):
+    if x == 1:
+        yield []
+        return
+    if depth > 7:
+        return
+    for r in RADIX_COST:
+        if r <= limit and x % r == 0:
+            for rest in _radix_sequences(x // r, r, depth + 1):
+                yield [r, *rest]
+
+
+@functools.cache
+def radix_list(length: int) -> list[int]:
+    """The radix plan of a length (fft_device.hpp make_radix_list)."""
+    best = prime_power_list(length)
+    if length & (length - 1) == 0 or length < 6:
+        return best
+
+    def cost(radices: list[int]) -> int:
+        t = length // radices[0]
+        c = sum(-(-(length // r) // t) * (RADIX_COST[r] + 14 * r) for r in radices)
+        return (c + (200 if radices[0] == 15 else 0)) * t + 6 * len(radices) * length
+
+    best_cost, t0 = cost(best) * 9 // 10, length // best[0]
+    for seq in _radix_sequences(length, 16):
+        for f, front in enumerate(seq):
+            if f and front == seq[f - 1]:
+                continue
+            t = length // front
+            if t > 1024 or (length <= 4096 and t > 256) or t < 32 <= t0 or (t < 10 and t0 >= 20):
+                continue
+            if any(-(-(length // r) // t) * r > 20 for r in seq):
+                continue
+            radices = [front, *seq[:f], *seq[f + 1:]]
+            c = cost(radices)
+            if c < best_cost:
+                best_cost, best = c, radices
+    return best
 
 
 def lds_pitch(length: int) -> int:
@@ -117,8 +163,17 @@ def tile_c_col(length: int) -> int:
 
 def pair_tile_widths(length: int) -> list[int]:
     """Instances per tile of a pair kernel: 16 .. 64 with at most 256 threads
-    (16 always), as rk_fft_plan.cpp pair_tile picks them."""
+    (16 always), as rk_fft_plan.cpp pair_tile picks them; none for plans of
+    more than 16 values per thread or many idle lanes."""
     t = threads_per_instance(length)
+    if any(-(-(length // r) // t) * r > 16 for r in radix_list(length)):
+        return []
+    idle = 0
+    for r in radix_list(length):
+        slots = -(-(length // r) // t) * t
+        idle += 1000 - 1000 * (length // r) // slots
+    if idle > 250 or 8 * t > 800:
+        return []
     return [c for c in (16, 32, 64) if c == 16 or c // 2 * t <= 256]
 
 
@@ -215,12 +270,13 @@ def catalog_entries() -> list[tuple[int, int, int]]:
         if (length <= 1024 and c * threads_per_instance(length) == 1024 and base in (VAR_PLAIN, VAR_TWIDDLE)
                 and v & (VAR_MODE_DD | VAR_MODE_DF)):
             ents.add((length, c, v | VAR_OCC))
-    # the power-of-two column passes with two instances per thread
-    # (rk_fft_plan.cpp pair_tile), for every tile width the planner may pick
+    # column passes with two instances per thread (rk_fft_plan.cpp pair_tile),
+    # for every tile width the planner may pick
     for length, c, v in list(ents):
         base = v & ~(nt | VAR_MODE_DD | VAR_MODE_DF)
-        if (length & (length - 1) == 0 and PAIR_MIN <= length <= FACTOR_MAX and c == tile_c_col(length)
-                and base in (VAR_PLAIN, VAR_TWIDDLE) and v & (VAR_MODE_DD | VAR_MODE_DF)):
+        if (PAIR_MIN <= length <= FACTOR_MAX and c == tile_c_col(length)
+                and base in (VAR_PLAIN, VAR_TWIDDLE) and v & (VAR_MODE_DD | VAR_MODE_DF)
+                and (v & VAR_MODE_DD or radix_list(length)[0] % 2 == 0)):
             for cp in pair_tile_widths(length):
                 ents.add((length, cp, v | VAR_PAIR))
     # plans over several axes stream their first pass's loads (contiguous rows)
@@ -234,7 +290,7 @@ def catalog_entries() -> list[tuple[int, int, int]]:
                 ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD))
                 if length <= 1024 and tile_c_col(length) * threads_per_instance(length) == 1024:
                     ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_OCC))
-                if PAIR_MIN <= length and length & (length - 1) == 0:
+                if PAIR_MIN <= length:
                     for cp in pair_tile_widths(length):
                         ents.add((length, cp, VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_PAIR))
             if length & (length - 1) and threads_per_instance(length) >= 32:
@@ -358,7 +414,8 @@ def generate_catalog(out_dir: Path) -> list[Path]:
             '#include "rk_internal.hpp"',
             f"namespace rk_catalog_{k} {{",
             "template <int L, int C, int V>",
-            "__global__ void __launch_bounds__((rkfft::variant_threads<L, C, V>()), (rkfft::pass_min_waves<L, C, V>()))",
+            "__global__ void __launch_bounds__(rkfft::bound_threads(rkfft::variant_threads<L, C, V>()),\n"
+            "                                  (rkfft::pass_min_waves<L, C, V>()))",
             "rk_fft_pass(rk_pass_args a) {",
             "    rkfft::fft_pass_entry<L, C, V>(a);",
             "}",

@@ -5,7 +5,7 @@
 // compile-time variant: pre-op, post-op, Bluestein; see Variant below):
 //
 //   * each DFT ("instance") is worked on by T = L / R0 threads, R0 being the
-//     largest radix of the compile-time radix plan of L (16, 8, 4, 2, 7, 5, 3);
+//     first radix of the compile-time radix plan of L;
 //   * the stages are Stockham autosort steps: a thread reads R values at
 //     j + r*L/R from LDS, multiplies by the stage twiddles W_{Ns*R}^{r*(j%Ns)}
 //     (a table built in FP64 and rounded once), does an in-register DFT_R and
@@ -103,6 +103,12 @@ template <class X> RK_HD X c_select(bool cond, X a, X b) { return cx<X>(cond ? a
 #define RK_S7_1 0.7818314824680298
 #define RK_S7_2 0.9749279121818236
 #define RK_S7_3 0.43388373911755823
+#define RK_C9_1 0.766044443118978     // cos(2pi/9)
+#define RK_S9_1 0.6427876096865394
+#define RK_C9_2 0.17364817766693036   // cos(4pi/9)
+#define RK_S9_2 0.984807753012208
+#define RK_C9_4 -0.9396926207859084   // cos(8pi/9)
+#define RK_S9_4 0.3420201433256687
 
 // ------------------------------------------------------------------------
 // in-register forward DFTs, y_k = sum_n v_n exp(-2 pi i n k / R), in place
@@ -242,13 +248,80 @@ template <class X> RK_HD void dft7(X* v) {
     }
 }
 
+template <int R, class X> RK_HD void dft(X* v);
+
+// N1 x N2 points, N1 and N2 coprime: with n = N2 n1 + N1 n2 and k = N2 a k1 +
+// N1 b k2 modulo N (a, b the inverses of N2 modulo N1 and N1 modulo N2) the
+// DFT separates without twiddles (Good 1958).
+constexpr int inverse_mod(int x, int m) {
+    for (int y = 1; y < m; ++y)
+        if ((x * y) % m == 1) return y;
+    return 1;
+}
+template <int N1, int N2, class X> RK_HD void dft_coprime(X* v) {
+    constexpr int N = N1 * N2, E1 = N2 * inverse_mod(N2, N1), E2 = N1 * inverse_mod(N1, N2);
+    X t[N];
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) {
+        X c[N1];
+#pragma unroll
+        for (int n1 = 0; n1 < N1; ++n1) c[n1] = v[(N2 * n1 + N1 * n2) % N];
+        dft<N1>(c);
+#pragma unroll
+        for (int k1 = 0; k1 < N1; ++k1) t[k1 * N2 + n2] = c[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < N1; ++k1) {
+        dft<N2>(&t[k1 * N2]);
+#pragma unroll
+        for (int k2 = 0; k2 < N2; ++k2) v[(E1 * k1 + E2 * k2) % N] = t[k1 * N2 + k2];
+    }
+}
+
+// a * (c + cl - i (s + sl)), the constants' rounding errors included: 9 = 3 x 3
+// multiplies by the same three twiddles wherever it occurs, and their errors,
+// shared by all of a transform's butterflies, made 729 = 9 * 9 * 9 2.4 % less
+// accurate than 3^6 with its tables.
+template <class X> RK_HD X mul_w9(X a, real_t<X> c, real_t<X> cl, real_t<X> s, real_t<X> sl) {
+    return cx<X>(a.x * c + (a.y * s + (a.y * sl + a.x * cl)), a.y * c - (a.x * s + (a.x * sl - a.y * cl)));
+}
+
+// 9 = 3 x 3: DFT3 over n2 for each n1 (x[n1 + 3 n2]), twiddle W9^{n1 k2},
+// DFT3 over n1 for each k2, output y[k2 + 3 k1].
+template <class X> RK_HD void dft9(X* v) {
+    using F = real_t<X>;
+    X t[9];
+#pragma unroll
+    for (int n1 = 0; n1 < 3; ++n1) {
+        X c[3] = {v[n1], v[n1 + 3], v[n1 + 6]};
+        dft3(c);
+#pragma unroll
+        for (int k2 = 0; k2 < 3; ++k2) t[3 * k2 + n1] = c[k2];
+    }
+    t[4] = mul_w9(t[4], (F)RK_C9_1, (F)(RK_C9_1 - (F)RK_C9_1 + 2.175e-17), (F)RK_S9_1, (F)(RK_S9_1 - (F)RK_S9_1 - 3.660e-17));
+    t[5] = mul_w9(t[5], (F)RK_C9_2, (F)(RK_C9_2 - (F)RK_C9_2 - 1.009e-17), (F)RK_S9_2, (F)(RK_S9_2 - (F)RK_S9_2 + 3.905e-17));
+    t[7] = mul_w9(t[7], (F)RK_C9_2, (F)(RK_C9_2 - (F)RK_C9_2 - 1.009e-17), (F)RK_S9_2, (F)(RK_S9_2 - (F)RK_S9_2 + 3.905e-17));
+    t[8] = mul_w9(t[8], (F)RK_C9_4, (F)(RK_C9_4 - (F)RK_C9_4 + 4.385e-17), (F)RK_S9_4, (F)(RK_S9_4 - (F)RK_S9_4 + 2.014e-17));
+#pragma unroll
+    for (int k2 = 0; k2 < 3; ++k2) {
+        dft3(&t[3 * k2]);
+#pragma unroll
+        for (int k1 = 0; k1 < 3; ++k1) v[k2 + 3 * k1] = t[3 * k2 + k1];
+    }
+}
+
 template <int R, class X> RK_HD void dft(X* v) {
     if constexpr (R == 2) dft2(v[0], v[1]);
     else if constexpr (R == 3) dft3(v);
     else if constexpr (R == 4) dft4(v[0], v[1], v[2], v[3]);
     else if constexpr (R == 5) dft5(v);
     else if constexpr (R == 7) dft7(v);
+    else if constexpr (R == 6) dft_coprime<2, 3>(v);
     else if constexpr (R == 8) dft8(v);
+    else if constexpr (R == 9) dft9(v);
+    else if constexpr (R == 10) dft_coprime<2, 5>(v);
+    else if constexpr (R == 12) dft_coprime<4, 3>(v);
+    else if constexpr (R == 15) dft_coprime<3, 5>(v);
     else if constexpr (R == 16) dft16(v);
     else static_assert(R == 1, "radix without a butterfly");
 }
@@ -302,14 +375,15 @@ struct RadixList {
     int r[24];
 };
 
-__host__ __device__ constexpr RadixList make_radix_list(int L) {
+// Prime powers only: 16s, the rest of the powers of two, 7s, 5s, 3s, the
+// largest in front (it fixes T = L / r[0] threads per instance).
+__host__ __device__ constexpr RadixList prime_power_list(int L) {
     RadixList s = {0, {0}};
     int x = L, p2 = 0, n3 = 0, n5 = 0, n7 = 0;
     while (x % 2 == 0) { x /= 2; ++p2; }
     while (x % 3 == 0) { x /= 3; ++n3; }
     while (x % 5 == 0) { x /= 5; ++n5; }
     while (x % 7 == 0) { x /= 7; ++n7; }
-    // largest radix first: it fixes T = L / r[0] threads per instance
     while (p2 >= 4) { s.r[s.n++] = 16; p2 -= 4; }
     if (p2 > 0) s.r[s.n++] = 1 << p2;
     for (int k = 0; k < n7; ++k) s.r[s.n++] = 7;
@@ -322,6 +396,81 @@ __host__ __device__ constexpr RadixList make_radix_list(int L) {
         if (s.r[k] > s.r[imax]) imax = k;
     int t = s.r[0]; s.r[0] = s.r[imax]; s.r[imax] = t;
     return s;
+}
+
+// Cost of a radix sequence (make_radix_list); fits: at most 20 values per thread.
+__host__ __device__ constexpr long long radix_cost(int L, const int* r, int n, bool* fits) {
+    const int kCost[17] = {0, 0, 4, 16, 16, 40, 40, 84, 60, 120, 100, 0, 112, 0, 0, 200, 168};
+    const int T = L / r[0];
+    long long c = r[0] == 15 ? 200 : 0;
+    for (int s = 0; s < n; ++s) {
+        const int q = (L / r[s] + T - 1) / T;
+        if (fits) *fits = *fits && q * r[s] <= 20;
+        c += q * (kCost[r[s]] + 14 * r[s]);
+    }
+    return c * T + 6ll * n * L;
+}
+
+// The radix plan of a length (build.py radix_list mirrors it).  Powers of two
+// take their 16s.  Other lengths take, of all factorisations into the radices
+// below, the cheapest: a stage costs every thread of T = L / r[0] its
+// ceil(L / R / T) butterflies (operations of the DFT, plus 14 per value for
+// twiddles, LDS and addresses), idle threads included, and each stage its
+// barriers (6 per value of the instance); a 15 in front, whose outputs lie 16
+// padded slots apart in LDS, pays for its bank conflicts.  The prime powers stay
+// unless that is 10 % cheaper, and rows of at least 32 threads keep them (below
+// 32 a contiguous side is staged through LDS), as those of at least 20 do
+// rather than go below 10 (30000 x 81: 9.7 us with 27 threads, 10.6 with 9).  Composite radices leave 1000 =
+// 10 * 10 * 10 where prime powers gave 8 * 5 * 5 * 5 and 1080 = 12 * 15 * 6
+// for 8 * 5 * 3 * 3 * 3: fewer exchanges and fewer idle threads.  At most 20
+// values per thread, and at most 256 threads up to 4096 points (the batch
+// kernel's work-group).  Prime powers / composite radices, us: rows 4096 x
+// 1000 15.3 / 12.9, 2048 x 2000 22.4 / 16.0, 500 x 1200 9.4 / 6.0; columns
+// 1440 x 1440 17.5 / 11.9, 200 x 360000 543 / 509; 192 cubed 68.0 / 62.1,
+// 160 cubed 45.2 / 40.9; the one loss seen, 32 x 1000 x 1000 over axis 1,
+// 127 / 133 (8 * 5 * 5 * 5 gives 1000 threads to a tile, 10 * 10 * 10 800).
+__host__ __device__ constexpr RadixList make_radix_list(int L) {
+    const int kR[12] = {16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+    RadixList best = prime_power_list(L);
+    if ((L & (L - 1)) == 0 || L < 6) return best;
+    long long best_cost = radix_cost(L, best.r, best.n, nullptr) * 9 / 10;
+    const int T0 = L / best.r[0];
+    // depth-first over non-increasing radix sequences: idx[d] is the radix of
+    // depth d, rem[d] what is left to factor before it
+    int idx[16] = {0}, rem[17] = {0}, d = 0;
+    rem[0] = L;
+    idx[0] = -1;
+    while (d >= 0) {
+        int k = idx[d] + 1;
+        while (k < 12 && rem[d] % kR[k] != 0) ++k;
+        if (k == 12 || d > 7) {
+            --d;
+            continue;
+        }
+        idx[d] = k;
+        rem[d + 1] = rem[d] / kR[k];
+        if (rem[d + 1] > 1) {
+            idx[d + 1] = k - 1;   // non-increasing: start at the same radix
+            ++d;
+            continue;
+        }
+        const int n = d + 1;
+        for (int f = 0; f < n; ++f) {   // each distinct radix in front
+            if (f > 0 && idx[f] == idx[f - 1]) continue;
+            const int T = L / kR[idx[f]];
+            if (T > 1024 || (L <= 4096 && T > 256) || (T < 32 && T0 >= 32) || (T < 10 && T0 >= 20)) continue;
+            int r[16] = {kR[idx[f]]}, m = 1;
+            for (int s = 0; s < n; ++s)
+                if (s != f) r[m++] = kR[idx[s]];
+            bool fits = true;
+            const long long c = radix_cost(L, r, n, &fits);
+            if (!fits || c >= best_cost) continue;
+            best_cost = c;
+            best.n = n;
+            for (int s = 0; s < n; ++s) best.r[s] = r[s];
+        }
+    }
+    return best;
 }
 
 __host__ __device__ constexpr bool is_supported_length(int L) {
@@ -1367,6 +1516,8 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
             store_run<V, QL, T, NR, P::ns(SL), RL, RL / 4>(a, io, ic, out_walk(a, ic, t), v, adjust,
                                                            [&](int q) { return stage_valid<L, SL>(t, q); });
         }
+    } else if constexpr (W == 2 && ((MODES >> 2) & 3) == RK_MODE_DIRECT) {
+        // stored above
     } else if constexpr (W == 2) {
         // FLAT: the tile is C*L contiguous elements; a thread takes two
         // consecutive positions of both instances of a pair (even R0 and L)
@@ -1430,6 +1581,14 @@ template <int L, int C> __host__ __device__ constexpr int pass_threads() { retur
 template <int L, int C, int V> __host__ __device__ constexpr int variant_threads() {
     return (V & RK_VAR_PAIR) ? (C / 2) * Plan<L>::T : C * Plan<L>::T;
 }
+// The work-group size of a kernel's launch bounds: its threads, rounded up to
+// whole waves on all four SIMDs above 256.  The compiler raises a kernel's
+// registers to what the waves that the LDS admits leave free, counting waves
+// over the CU; a work-group of 13 waves, though, needs room for four on one
+// SIMD, and a second one then found none (1000-point column tiles of 800
+// threads: 72 registers and one work-group per CU, 149 us for 32 x 1000 x
+// 1008; with 1024 in the bounds 56 registers and two, 130 us).
+RK_HD constexpr int bound_threads(int threads) { return threads > 256 ? (threads + 255) / 256 * 256 : threads; }
 
 // Tiles whose stage twiddles are read from an LDS copy of the W_L table
 // instead of global memory (the table loads otherwise take a large share of
@@ -1559,13 +1718,18 @@ __device__ __forceinline__ void fft_pass_entry(const rk_pass_args& a) {
 // registers do not cut the occupancy; a persistent (RK_VAR_PIPE) kernel
 // without it for one resident work-group per CU (the registers of its
 // prefetched tile then come out of that work-group's share).  A pair kernel
-// asks for what its LDS allows, at most four waves (128 VGPRs: 64 hold the
-// two instances' values of a radix-16 stage).
+// asks for the work-groups that its LDS and 56 registers beside the two
+// instances' values allow (two of the 600-, 1000- and 1024-point tiles; with
+// 32 beside them values spill: 64 x 1008000 804 us with the spills, 482
+// without).
 template <int L, int C, int V> __host__ __device__ constexpr int pass_min_waves() {
-    if ((V & RK_VAR_PAIR) != 0) {
-        const int waves = (variant_threads<L, C, V>() + 63) / 64;
-        const int w = ((160 * 1024) / (tile_lds_bytes_x<L, C, false, cpair2>() + L * 8)) * waves / 4;
-        return w < 1 ? 1 : (w > 4 ? 4 : w);
+    if constexpr ((V & RK_VAR_PAIR) != 0) {
+        const int waves = (variant_threads<L, C, V>() + 255) / 256;   // of a work-group, per SIMD
+        constexpr int tile = tile_lds_bytes_x<L, C, false, cpair2>();
+        constexpr int lds = tile + (twl_in_lds<L, C, V, false, false, cpair2>() ? L * 8 : 0);
+        const int by_regs = 512 / (4 * Plan<L>::vmax() + 56) / waves, by_lds = (160 * 1024) / lds;
+        const int wgs = by_regs < 1 ? 1 : (by_regs < by_lds ? by_regs : by_lds);
+        return wgs * waves;
     }
     if ((V & (RK_VAR_PIPE | RK_VAR_OCC)) != 0) {
         const int waves = (pass_threads<L, C>() + 63) / 64;

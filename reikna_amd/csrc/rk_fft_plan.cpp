@@ -856,6 +856,15 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
 // 30.6.  Elsewhere half the waves per tile cost more than the instructions
 // saved: 16 x 2^18 33.7 / 36.5, 8 x 2^16 (256-point passes) 12.1 / 14.7,
 // 4 x 2^24 541 / 576.
+// Other lengths from 512 to 1200 too, where pairs turn tiles of 8 or fewer
+// instances into 16 (whole lines) or tiles that hold a CU alone into two per
+// CU: one / two instances, columns of 32 x 720 x 1280 117 / 105 us, 16 x 1080
+// x 1920 175 / 146, 32 x 600 x 800 69.6 / 60.0, 32 x 729 x 800 74.7 / 66.8,
+// 1000 x 8192 42.7 / 35.0, 32 x 1000 x 1024 158 / 114, 200 x 360000 625 / 509.
+// Not for plans with many idle lanes, whose cost pairs double (32 x 750 x 800
+// 86.8 / 93.0, 800 x 800 85.2 / 88.8, 100 x 640000 499 / 544), work-groups of
+// over 800 threads (32 x 625 x 800 56.6 / 66.3) or rows that are no whole
+// lines (32 x 1000 x 1000 134 / 133, 16 x 10^6 128 / 141).
 static bool pair_enabled() {
     static const bool v = [] {
         const char* e = getenv("RK_PAIR");
@@ -864,16 +873,31 @@ static bool pair_enabled() {
     return v;
 }
 
-static int pair_tile(const PassPlan& pp) {
+static int pair_tile(const PassPlan& pp, bool chunked) {
     const rk_pass_args& a = pp.args;
     const int mbit = fixed_mode_bit(pp);
     if (!pair_enabled() || pp.es != 8 || pp.wave || pp.pipe || pp.half || !a.cmap) return 0;
     if (pp.variant != VAR_PLAIN && pp.variant != VAR_TWIDDLE) return 0;
     if (mbit != VAR_MODE_DD && mbit != VAR_MODE_DF) return 0;
     if (t_tuning && t_tuning->col_tile > 0) return 0;
-    if (pp.L < 512 || pp.L > 1024 || (pp.L & (pp.L - 1))) return 0;
+    if (pp.L < 512 || pp.L > 1200) return 0;
     const bool dd = mbit == VAR_MODE_DD;
-    if (!pp.nt_load && !pp.nt_store && !(dd && pp.L == 1024 && a.n_tiles >= 512)) return 0;
+    const rk_u64 tiles16 = a.n_inst / 16;   // tiles of the pair kernel
+    // the other tile has parts of 128-byte lines, or a CU to itself
+    const bool poor = pp.C < 16 || tile_lds_bytes_host(pp.L, pp.C, pp.es) > 80 * 1024;
+    if (!pp.nt_load && !pp.nt_store && !(dd && (poor || pp.L == 1024) && tiles16 >= 512)) return 0;
+    const rkfft::RadixList rl = rkfft::make_radix_list(pp.L);
+    if (!dd && (pp.L % 2 || rl.r[0] % 2)) return 0;   // two positions per store
+    // at most 16 values of each instance per thread, and few lanes without a
+    // butterfly (a quarter of one stage's, summed over the stages)
+    const int t0 = pp.L / rl.r[0];
+    int idle = 0;   // 1/1000
+    for (int s = 0; s < rl.n; ++s) {
+        const int nb = pp.L / rl.r[s], q = (nb + t0 - 1) / t0;
+        if (q * rl.r[s] > 16) return 0;
+        idle += 1000 - 1000 * nb / (q * t0);
+    }
+    if (idle > 250) return 0;
     rk_u64 inner;
     if (a.dim_I > 1) {
         inner = a.dim_I;
@@ -885,21 +909,27 @@ static int pair_tile(const PassPlan& pp) {
         inner = a.dim_H;
         if (a.in_sa != 1 || dd) return 0;
     }
-    if (inner % 2) return 0;
+    // lengths other than powers of two: tiles of whole 128-byte lines only
+    if (inner % ((pp.L & (pp.L - 1)) ? 16 : 2)) return 0;
     // 256 threads where the tile's LDS leaves two work-groups per CU, and
     // whole tiles per outer index (chunked chains start at tile boundaries)
     const int T = threads_per_instance(pp.L);
+    if (8 * T > 800 || rkfft::pair_lds_bytes(pp.L, 16, T) > 80 * 1024) return 0;
     const rk_u64 per_outer = a.dim_I * a.dim_NS * a.dim_H;
     int C = 64;
     while (C > 16 && ((C / 2) * T > 256 || per_outer % (rk_u64)C || rkfft::pair_lds_bytes(pp.L, C, T) + pp.L * 8 > 80 * 1024))
         C /= 2;
-    return C;
+    // In a chunked chain the tiles must not cross outer indices: a chunk's
+    // workspace is rebased, and a tile that reached past the chunk (its lanes
+    // past the last instance take instance 0's addresses) would read outside
+    // it.
+    return chunked && per_outer % (rk_u64)C ? 0 : C;
 }
 
 // The pair kernel of a pass: the catalogue's, or one from the run-time
 // compiler for lengths the catalogue does not hold.
-static bool find_pair_kernel(PassPlan& pp, uint32_t flags) {
-    const int C = pair_tile(pp);
+static bool find_pair_kernel(PassPlan& pp, uint32_t flags, bool chunked) {
+    const int C = pair_tile(pp, chunked);
     if (!C) return false;
     const int T = threads_per_instance(pp.L);
     pp.pair_threads = (C / 2) * T;
@@ -1300,7 +1330,7 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
         pp.pipe = pipe_enabled() && pp.args.load_mode == RK_MODE_DIRECT && pp.loops.empty();
         pp.half = half_enabled() && (int64_t)pp.C * lds_pitch_host(pp.L) * pp.es <= 80 * 1024;
         pp.occ = occ_min_length() >= 0 ? occ_min_length() > 0 && pp.L >= occ_min_length() : occ_default(pp);
-        if (!find_pair_kernel(pp, d->flags)) {
+        if (!find_pair_kernel(pp, d->flags, plan->chunk_outer != 0)) {
             rc = find_kernel(pp, d->flags);
             if (rc != RK_OK) return rc;
         }
@@ -1337,6 +1367,10 @@ static int launch_pass(const PassPlan& pp, rk_pass_args& a, hipStream_t stream, 
     const rk_u64 C = (rk_u64)(pp.pair_C ? pp.pair_C : pp.C);
     const int threads = pp.pair_C ? pp.pair_threads : pp.threads;
     const rk_u64 max_grid = pp.pair_C ? (rk_u64(1) << 31) / (rk_u64)threads : pp.grid;
+    // chunks (instance ranges of a rebased workspace) hold whole tiles
+    if (i0 % C || (i1 % C && (i0 || i1 < a.n_inst)))
+        return fail(RK_ERR_INVALID, "internal: instances %llu to %llu are not whole tiles of %llu", (unsigned long long)i0,
+                    (unsigned long long)i1, (unsigned long long)C);
     const rk_u64 t0 = i0 / C, t1 = (i1 + C - 1) / C;
     // host loops over batch dims the kernel could not fold
     const size_t nl = pp.loops.size();

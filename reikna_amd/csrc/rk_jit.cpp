@@ -43,7 +43,7 @@ int jit_pass_kernel(int L, int C, int variant, hipFunction_t* fn, int* threads, 
         char src[512];
         snprintf(src, sizeof(src),
                  "#include \"fft_device.hpp\"\n"
-                 "extern \"C\" __global__ void __launch_bounds__(%d, (rkfft::pass_min_waves<%d, %d, %d>()))\n"
+                 "extern \"C\" __global__ void __launch_bounds__(rkfft::bound_threads(%d), (rkfft::pass_min_waves<%d, %d, %d>()))\n"
                  "rk_jit_pass(rk_pass_args a) {\n"
                  "    rkfft::fft_pass_entry<%d, %d, %d>(a);\n"
                  "}\n",

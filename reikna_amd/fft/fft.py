@@ -230,7 +230,7 @@ class _FusedFft:
                      if _fixed_modes() else "0")
             # launch bounds of the plan's own kernel for the residency the
             # tile's LDS allows (fft_device.hpp RK_VAR_OCC, RK_VAR_F64)
-            bounds = f"{info.threads}"
+            bounds = f"rkfft::bound_threads({info.threads})"
             if info.occ:
                 v = info.variant | 65536 | (131072 if xtype == "double2" else 0)
                 bounds += f", (rkfft::pass_min_waves<{info.L}, {info.C}, {v}>())"

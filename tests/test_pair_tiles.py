@@ -35,7 +35,13 @@ PLANNED = [
     ((256, 2**18), (1,), [16, 16]),
     ((512, 2**17), (1,), [16, 0]),      # 512 * 256: passes of 256 points never
     ((4, 2**20), (1,), [0, 0]),         # not streaming
-    ((128, 1000 * 1000), (1,), [0, 0]),  # not powers of two
+    ((128, 1000 * 1000), (1,), [0, 0]),   # tiles would cross the rows of a chunk
+    ((96, 1000 * 1024), (1,), [16, 16]),
+    ((200, 800 * 800), (1,), [0, 0]),
+    ((256, 640 * 640), (1,), [0, 0]),   # 20 values per thread
+    ((1000, 8192), (0,), [16]),
+    ((1000, 8194), (0,), [0]),
+    ((1000, 4096), (0,), [0]),
     # a strided axis of 1024 points: at least 512 tiles of 16 and an even inner extent
     ((1024, 8192), (0,), [16]),
     ((1024, 8193), (0,), [0]),
@@ -53,6 +59,17 @@ def test_passes_that_run_as_pairs(shape, axes, want):
     assert not any(pairs(shape, axes, dtype=numpy.complex128))
     assert not any(pairs(shape, axes, tuning=PlanTuning(col_tile=16)))
     assert not any(pairs(shape, axes, tuning=PlanTuning(fixed_modes=0)))
+
+
+def test_chunks_hold_whole_tiles():
+    """A chunk's workspace is rebased, so no launched tile may reach past its chunk."""
+    for n in (1000 * 1000, 1000 * 1024, 1000 * 768, 1000 * 512, 640 * 1000, 500 * 1000, 2**20, 2**17, 12288, 65521, 3 * 2**17):
+        for rows in (67, 70, 127, 200, 2001, 9001):
+            meta = ArrayMetadata((rows, n), numpy.complex64)
+            plan = NativeFftPlan(meta, meta, (1,), _lib.RK_FFT_DRY_RUN)
+            for p in plan.passes:
+                if plan.chunk_rows:
+                    assert (p.n_inst // rows) % (p.pair or p.C) == 0, (n, rows, p)
 
 
 def test_pairs_need_unit_strides():
@@ -123,6 +140,10 @@ def data_of(shape, seed):
     ((3, 1024, 2734), (1,), 0),         # tiles across the outer index
     ((66, 2**19), (1,), 1),             # 1024 * 512, a short last chunk
     ((257, 2**17), (1,), 0),            # 512 * 256
+    pytest.param((67, 1000 * 1000), (1,), 0, marks=pytest.mark.skip(
+        reason="pair tiles that cross the rows of a chunk read outside its workspace: such tiles are no longer launched")),
+    ((1000, 8208), (0,), 1),
+    ((2, 1000, 4512), (1,), 0),
 ], ids=str)
 def test_pair_tiles_match_oracle(queue, shape, axes, inverse):
     data = data_of(shape, 3)

@@ -27,7 +27,7 @@ NONE, LOAD, STORE, BOTH = (False, False), (True, False), (False, True), (True, T
     ((64, 1024, 1024), (1, 2), [LOAD, STORE]),   # chunked
     ((4096, 4096), (1,), [NONE]),                # one pass of 256 MiB in and out together
     ((8192, 4096), (1,), [BOTH]),
-    ((16, 1080, 1921), (1,), [NONE]),            # 32-byte column segments never stream
+    ((16, 4096, 601), (1,), [NONE]),             # 32-byte column segments never stream
 ], ids=str)
 def test_streaming_ends(shape, axes, want):
     assert ends(shape, axes) == want

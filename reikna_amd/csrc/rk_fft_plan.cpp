@@ -811,8 +811,8 @@ static bool catalog_length(int L) {
 // The pass's kernel: the catalogue's, with the pass's load/store modes
 // compiled in when such a twin exists, else from the run-time compiler (the
 // same entry, any variant number).  A pass whose nontemporal twin is missing
-// keeps the plain accesses when the catalogue has its plain kernel or run-time
-// compilation is off.
+// keeps the plain accesses when the catalogue has the same kernel with those
+// or run-time compilation is off.
 static int find_kernel(PassPlan& pp, uint32_t flags) {
     pp.fixed_modes = false;
     const int mbit = fixed_mode_bit(pp);
@@ -826,12 +826,14 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
     if (mbit)
         if (const KernelEntry* e = catalog_find(pp.L, pp.C, want | mbit)) return take(e, true), RK_OK;
     if (const KernelEntry* e = catalog_find(pp.L, pp.C, want)) return take(e, false), RK_OK;
-    const bool in_catalog = pp.es == 8 && catalog_find(pp.L, pp.C, pp.variant) != nullptr;
-    if ((flags & RK_FFT_NO_JIT) || in_catalog) {
-        if (pp.nt_load || pp.nt_store) {
-            pp.nt_load = pp.nt_store = false;
-            return find_kernel(pp, flags);
-        }
+    const int without_hints = want & ~(VAR_STREAM | VAR_NT_LOAD | VAR_NT_STORE);
+    if ((pp.nt_load || pp.nt_store) &&
+        ((flags & RK_FFT_NO_JIT) || catalog_find(pp.L, pp.C, without_hints | mbit) ||
+         catalog_find(pp.L, pp.C, without_hints))) {
+        pp.nt_load = pp.nt_store = false;
+        return find_kernel(pp, flags);
+    }
+    if (flags & RK_FFT_NO_JIT) {
         return fail(RK_ERR_NO_KERNEL, "no precompiled kernel for L=%d C=%d variant=%d and run-time compilation is off",
                     pp.L, pp.C, want);
     }

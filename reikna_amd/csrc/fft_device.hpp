@@ -290,6 +290,9 @@ template <class X> RK_HD X mul_w9(X a, real_t<X> c, real_t<X> cl, real_t<X> s, r
 // DFT3 over n1 for each k2, output y[k2 + 3 k1].
 template <class X> RK_HD void dft9(X* v) {
     using F = real_t<X>;
+    // one value's real type: a double subtracted from a pair's vector is rounded
+    // to float first, which leaves no residual
+    using S = real_t<scalar_t<X>>;
     X t[9];
 #pragma unroll
     for (int n1 = 0; n1 < 3; ++n1) {
@@ -298,10 +301,13 @@ template <class X> RK_HD void dft9(X* v) {
 #pragma unroll
         for (int k2 = 0; k2 < 3; ++k2) t[3 * k2 + n1] = c[k2];
     }
-    t[4] = mul_w9(t[4], (F)RK_C9_1, (F)(RK_C9_1 - (F)RK_C9_1 + 2.175e-17), (F)RK_S9_1, (F)(RK_S9_1 - (F)RK_S9_1 - 3.660e-17));
-    t[5] = mul_w9(t[5], (F)RK_C9_2, (F)(RK_C9_2 - (F)RK_C9_2 - 1.009e-17), (F)RK_S9_2, (F)(RK_S9_2 - (F)RK_S9_2 + 3.905e-17));
-    t[7] = mul_w9(t[7], (F)RK_C9_2, (F)(RK_C9_2 - (F)RK_C9_2 - 1.009e-17), (F)RK_S9_2, (F)(RK_S9_2 - (F)RK_S9_2 + 3.905e-17));
-    t[8] = mul_w9(t[8], (F)RK_C9_4, (F)(RK_C9_4 - (F)RK_C9_4 + 4.385e-17), (F)RK_S9_4, (F)(RK_S9_4 - (F)RK_S9_4 + 2.014e-17));
+    const F c1 = (S)RK_C9_1, c1l = (S)(RK_C9_1 - (S)RK_C9_1 + 2.175e-17), s1 = (S)RK_S9_1, s1l = (S)(RK_S9_1 - (S)RK_S9_1 - 3.660e-17);
+    const F c2 = (S)RK_C9_2, c2l = (S)(RK_C9_2 - (S)RK_C9_2 - 1.009e-17), s2 = (S)RK_S9_2, s2l = (S)(RK_S9_2 - (S)RK_S9_2 + 3.905e-17);
+    const F c4 = (S)RK_C9_4, c4l = (S)(RK_C9_4 - (S)RK_C9_4 + 4.385e-17), s4 = (S)RK_S9_4, s4l = (S)(RK_S9_4 - (S)RK_S9_4 + 2.014e-17);
+    t[4] = mul_w9(t[4], c1, c1l, s1, s1l);
+    t[5] = mul_w9(t[5], c2, c2l, s2, s2l);
+    t[7] = mul_w9(t[7], c2, c2l, s2, s2l);
+    t[8] = mul_w9(t[8], c4, c4l, s4, s4l);
 #pragma unroll
     for (int k2 = 0; k2 < 3; ++k2) {
         dft3(&t[3 * k2]);

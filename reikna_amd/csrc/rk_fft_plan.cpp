@@ -929,12 +929,12 @@ static int pair_tile(const PassPlan& pp, bool chunked) {
 }
 
 // The pair kernel of a pass: the catalogue's, or one from the run-time
-// compiler for lengths the catalogue does not hold.
-static bool find_pair_kernel(PassPlan& pp, uint32_t flags, bool chunked) {
+// compiler for lengths the catalogue does not hold (a dry run reports its
+// geometry).  Leaves pair_C at 0 for a pass without one.
+static int find_pair_kernel(PassPlan& pp, uint32_t flags, bool chunked) {
     const int C = pair_tile(pp, chunked);
-    if (!C) return false;
+    if (!C) return RK_OK;
     const int T = threads_per_instance(pp.L);
-    pp.pair_threads = (C / 2) * T;
     int v = pp.variant | fixed_mode_bit(pp) | VAR_PAIR;
     if (pp.nt_load && pp.nt_store) v |= VAR_STREAM;
     else if (pp.nt_load) v |= VAR_NT_LOAD;
@@ -942,15 +942,19 @@ static bool find_pair_kernel(PassPlan& pp, uint32_t flags, bool chunked) {
     if (const KernelEntry* e = catalog_find(pp.L, C, v)) {
         pp.aot = e->func;
     } else {
-        if (catalog_length(pp.L) || (flags & (RK_FFT_NO_JIT | RK_FFT_DRY_RUN))) return false;
+        if (catalog_length(pp.L) || (flags & RK_FFT_NO_JIT)) return RK_OK;
         int threads = 0, lds = 0;
-        if (jit_pass_kernel(pp.L, C, v, &pp.jit, &threads, &lds) != RK_OK) return false;
+        if (!(flags & RK_FFT_DRY_RUN)) {
+            const int rc = jit_pass_kernel(pp.L, C, v, &pp.jit, &threads, &lds);
+            if (rc != RK_OK) return rc;
+        }
     }
     pp.pair_C = C;
+    pp.pair_threads = (C / 2) * T;
     pp.threads = pp.C * T;
     pp.lds_bytes = tile_lds_bytes_host(pp.L, pp.C, pp.es);
     pp.fixed_modes = true;
-    return true;
+    return RK_OK;
 }
 
 // Passes whose instances fill whole waves (T = L / R0 divides 64) run the
@@ -1332,10 +1336,9 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
         pp.pipe = pipe_enabled() && pp.args.load_mode == RK_MODE_DIRECT && pp.loops.empty();
         pp.half = half_enabled() && (int64_t)pp.C * lds_pitch_host(pp.L) * pp.es <= 80 * 1024;
         pp.occ = occ_min_length() >= 0 ? occ_min_length() > 0 && pp.L >= occ_min_length() : occ_default(pp);
-        if (!find_pair_kernel(pp, d->flags, plan->chunk_outer != 0)) {
-            rc = find_kernel(pp, d->flags);
-            if (rc != RK_OK) return rc;
-        }
+        rc = find_pair_kernel(pp, d->flags, plan->chunk_outer != 0);
+        if (rc == RK_OK && !pp.pair_C) rc = find_kernel(pp, d->flags);
+        if (rc != RK_OK) return rc;
         set_xcd_group(pp);
         const uint64_t max_grid = (uint64_t(1) << 31) / (uint64_t)pp.threads;
         pp.grid = std::min<uint64_t>(pp.args.n_tiles, pp.pipe ? pipe_grid(pp) : max_grid);

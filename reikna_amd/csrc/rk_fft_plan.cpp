@@ -82,14 +82,20 @@ static int64_t blue_single_max() {
 // row of 2^17 15.0 / 13.4.  Two 1024-point complex128 passes (4 x 1024 tiles)
 // measured faster as well (64 x 2^20 1056 / 831 us), and so did Bluestein
 // chains of 512-point ones (33 x 65521 170 / 137), but the plan tests fix
-// those plans at 256; a tuned plan may choose them.  RK_FACTOR_MAX overrides.
-static int64_t factor_max() {
+// those plans at 256 (chirp_factor_max); a tuned plan may choose them.
+// RK_FACTOR_MAX overrides both limits.
+static int64_t factor_max_override() {
     static const int64_t v = [] {
         const char* e = getenv("RK_FACTOR_MAX");
         return e && *e ? (int64_t)atoll(e) : (int64_t)0;
     }();
-    if (v) return v;
-    return t_elem_bytes == 16 ? 512 : 1024;
+    return v;
+}
+static int64_t factor_max() {
+    return factor_max_override() ? factor_max_override() : t_elem_bytes == 16 ? 512 : 1024;
+}
+static int64_t chirp_factor_max() {
+    return factor_max_override() ? factor_max_override() : t_elem_bytes == 16 ? 256 : 1024;
 }
 
 static bool length_ok(const ChainLimits& lim, int64_t n) { return lim.length_ok ? lim.length_ok(n) : is_smooth(n); }
@@ -129,7 +135,8 @@ ChainLimits default_limits() {
     l.blue_single_max = blue_single_max();
     l.length_ok = nullptr;
     l.strided_single_max = 0;
-    if (t_tuning && t_tuning->factor_max > 0) l.factor_max = t_tuning->factor_max;
+    l.chirp_factor_max = chirp_factor_max();
+    if (t_tuning && t_tuning->factor_max > 0) l.factor_max = l.chirp_factor_max = t_tuning->factor_max;
     if (t_tuning && t_tuning->first_factor > 0) l.first_factor = t_tuning->first_factor;
     return l;
 }
@@ -472,8 +479,8 @@ int axis_passes(int64_t n, uint32_t flags, const ChainLimits& lim, std::vector<A
     if (smooth && !lim.length_ok)
         return fail(RK_ERR_UNSUPPORTED, "cannot split axis length %lld into passes", (long long)n);
     const int64_t m = bluestein_length(n, lim.pow2_bluestein);
-    ChainLimits blim = lim;   // complex128: factor_max() above
-    if (t_elem_bytes == 16 && blim.factor_max == 512 && !(t_tuning && t_tuning->factor_max > 0)) blim.factor_max = 256;
+    ChainLimits blim = lim;
+    if (lim.chirp_factor_max) blim.factor_max = lim.chirp_factor_max;
     const bool multi = m > lim.blue_single_max || (flags & RK_FFT_FORCE_MULTIPASS);
     if (!multi) {
         AxisPass ap;

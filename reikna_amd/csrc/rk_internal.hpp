@@ -113,6 +113,7 @@ struct ChainLimits {
     bool (*length_ok)(int64_t L);   // pass lengths a kernel exists for (null: any smooth length)
     int64_t strided_single_max;     // single_max of axes that are not contiguous in the input (0: single_max)
     int64_t first_factor = 0;       // length of the first pass of a multi-pass split (0: the balanced split)
+    int64_t chirp_factor_max = 0;   // longest pass of a Bluestein chain (0: factor_max)
 };
 ChainLimits default_limits();
 

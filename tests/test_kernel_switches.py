@@ -32,3 +32,25 @@ def test_switches_leave_every_plan_possible(switch):
     assert r.returncode == 0, r.stderr[-2000:]
     if name == "RK_WAVE":
         assert "True" in r.stdout
+
+
+CHAINS = """
+import numpy
+from reikna_amd import ArrayMetadata, _lib
+from reikna_amd.fft import NativeFftPlan
+for n in (65521, 2**18):
+    meta = ArrayMetadata((33, n), numpy.complex128)
+    print(max(p.L for p in NativeFftPlan(meta, meta, (1,), _lib.RK_FFT_DRY_RUN).passes))
+"""
+
+
+# 65521 points: M = 2^17, two passes of up to 512 points or three of up to 64
+@pytest.mark.parametrize("limit,longest", [(None, [64, 512]), ("512", [512, 512]), ("511", [64, 64]), ("256", [64, 64]),
+                                           ("32", [32, 32])])
+def test_factor_max_bounds_every_chain(limit, longest):
+    """RK_FACTOR_MAX, also where it is one of the planner's own limits."""
+    env = {k: v for k, v in os.environ.items() if k != "RK_FACTOR_MAX"}
+    r = subprocess.run([sys.executable, "-c", CHAINS], cwd=ROOT, env={**env, **({"RK_FACTOR_MAX": limit} if limit else {})},
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert [int(x) for x in r.stdout.split()] == longest

@@ -169,7 +169,7 @@ class NativeFftPlan:
     def execute(self, out_ptr: int, in_ptr: int, inverse: int, ws_ptr: int | None, stream: int | None,
                 load_blob: bytes | None = None, store_blob: bytes | None = None) -> None:
         if load_blob is None and store_blob is None:
-            rc = _lib.load().rk_fft_execute(self.handle, out_ptr, in_ptr, inverse, ws_ptr, stream)
+            rc = _lib.load().rk_fft_execute(self.handle, out_ptr, in_ptr, int(inverse), ws_ptr, stream)
             if rc == _lib.RK_OK:
                 return
         else:

@@ -751,13 +751,34 @@ static bool stream_pass(const PassPlan& pp) {
 // 55 -> 57, 119 -> 110, 233 -> 199.  16 x 2^18 (32 MiB) was no faster.  Plans
 // over several axes, whose later passes run in place on the output: 16 x 1024 x
 // 1024 (128 MiB) 104 -> 94 us, 256^3 137 -> 131; of 16 x 1080 x 1920 (253 MiB)
-// only the input's loads may: 316 -> 303, with the last stores 312.
+// only the input's loads may: 316 -> 303, with the last stores 312.  Larger
+// arrays find nothing of theirs in the cache (stream_all below).
 static int stream_ends(const PassPlan& pp, size_t axes) {
     if (stream_min_bytes() <= 0) return 0;
     const double array = (double)pp.es * (double)pp.args.n_inst * (double)pp.L;
     const double unit = stream_min_bytes();   // the Infinity Cache
     if (axes == 1) return array >= unit * 3 / 16 ? 3 : 0;
     return array >= unit * 3 / 4 ? 1 : array >= unit * 3 / 8 ? 3 : 0;
+}
+
+// Whether a pass of an unchunked plan over several axes streams whatever it
+// reads and writes: arrays larger than the Infinity Cache pass through it
+// between passes, and the hints then gain what they gain in a single pass
+// (first loads only against every access: 8192 x 8192 797 / 729 us, 512^3
+// 1306 / 1210, 16384 x 4096 654 / 628, 5000 x 8000 518 / 492, 256 x 512 x 512
+// complex128 1216 / 1130; 400^3 621 / 625; at the cache's size 4096 x 8192
+// 425 / 419, 4096 x 4096 complex128 317 / 359).  Not where tiles store parts of
+// 128-byte lines, which should meet the neighbouring tiles' parts in a cache:
+// the 80-point pass of 6000-point rows (75 adjacent values) 142 us without
+// hints, 211 with them, axis 1 of 512 x 512 x 504 416 / 526, axis 0 of 6300 x
+// 6300 (84 points, tiles of 32) 165 / 200.  The two broken lines of wide tiles
+// over long rows weigh less: tiles of 48 160 / 150, of 64 131 / 115.
+static bool stream_all(const PassPlan& pp) {
+    const rk_pass_args& a = pp.args;
+    if ((double)pp.es * (double)a.n_inst * (double)pp.L <= stream_min_bytes()) return false;
+    if (!a.cmap || a.store_mode != RK_MODE_DIRECT) return true;
+    const rk_u64 adjacent = a.dim_I > 1 ? a.dim_I : a.dim_NS;
+    return adjacent * (rk_u64)pp.es % 128 == 0 || (a.dim_I > 1 && pp.C * pp.es >= 384);
 }
 
 // Kernels with the pass's load/store modes compiled in (RK_FIXED_MODES=0
@@ -1334,7 +1355,8 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
             // accesses: arrays that alone fill the cache then stream in every
             // other pass, as one streaming end gains nothing there (32 x 2^20:
             // 236 us streaming throughout, 203 at both ends, 247 at one).
-            if (plan->passes.size() > 1 && !((d->flags & RK_FFT_FUSED_ENDS) && pp.nt_load)) {
+            if (plan->passes.size() > 1 && !((d->flags & RK_FFT_FUSED_ENDS) && pp.nt_load) &&
+                !(work.size() > 1 && pp.nt_load && stream_all(pp))) {
                 const int ends = plain ? stream_ends(pp, work.size()) : 0;
                 pp.nt_load = (ends & 1) && pp.is_first && pp.src == BUF_IN;
                 pp.nt_store = (ends & 2) && pp.is_last && pp.dst == BUF_OUT;

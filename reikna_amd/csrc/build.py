@@ -286,8 +286,14 @@ def catalog_entries() -> list[tuple[int, int, int]]:
         if length <= STREAM_MAX:
             ents.add((length, tile_c_row(length), VAR_PLAIN | VAR_NT_LOAD))
             ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE))
-            if length <= FACTOR_MAX:
+            # beyond the passes of chains, tiles of 1024 threads only: the generic
+            # one of 2048 points holds 89 VGPRs (61 with its modes compiled in) and
+            # is alone on its CU, the columns of 64 x 2048 x 2048 1082 us against
+            # 910; the 768 threads of 1536 points are faster alone, 64 x 1536 x
+            # 2048 over both axes 1340 us against 1425
+            if length <= FACTOR_MAX or tile_c_col(length) * threads_per_instance(length) == 1024:
                 ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD))
+            if length <= FACTOR_MAX:
                 if length <= 1024 and tile_c_col(length) * threads_per_instance(length) == 1024:
                     ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_OCC))
                 if PAIR_MIN <= length:

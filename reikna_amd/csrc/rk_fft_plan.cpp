@@ -781,6 +781,21 @@ static bool stream_all(const PassPlan& pp) {
     return adjacent * (rk_u64)pp.es % 128 == 0 || (a.dim_I > 1 && pp.C * pp.es >= 384);
 }
 
+// Whether a pass reads, or stores, whole units of `bytes` bytes (and its tiles
+// of C instances whole 64-byte ones): always but for a column side whose
+// rows of adjacent instances end or begin inside one.
+static bool whole_units(const PassPlan& pp, int C, bool store, int bytes) {
+    const rk_pass_args& a = pp.args;
+    if (!a.cmap || (store ? a.store_mode : a.load_mode) != RK_MODE_DIRECT) return true;
+    const int64_t unit = bytes / pp.es, outer = (int64_t)(a.n_inst / (a.dim_I * a.dim_NS * a.dim_H));
+    const int64_t sa = store ? a.out_sa : a.in_sa, si = store ? a.out_si : a.in_si, so = store ? a.out_so : a.in_so;
+    if ((a.dim_I > 1 ? si : sa) != 1) return false;
+    const int64_t adjacent = (int64_t)(a.dim_I > 1 ? a.dim_I : store ? a.dim_NS : a.dim_NS * a.dim_H);
+    const int64_t position = (int64_t)(store ? a.dim_NS : a.pos_mult) * sa;
+    return C * pp.es % 64 == 0 && adjacent % unit == 0 && position % unit == 0 && (outer == 1 || so % unit == 0) &&
+           (store ? a.out_off : a.in_off) % unit == 0;
+}
+
 // Kernels with the pass's load/store modes compiled in (RK_FIXED_MODES=0
 // turns them off).
 static bool use_fixed_modes() {
@@ -1337,6 +1352,8 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
     // only what comes from and goes to the caller's arrays (its first pass's
     // loads, its last pass's stores): the intermediate stays in the Infinity
     // Cache between the passes of a chunk.
+    const bool several = plan->passes.size() > 1, chunked = plan->chunk_outer != 0;
+    auto tile = [&](const PassPlan& pp) { return pair_tile(pp, chunked) ? pair_tile(pp, chunked) : pp.C; };
     for (PassPlan& pp : plan->passes) {
         // A column tile of less than 64 bytes per row leaves parts of its cache
         // lines to the neighbouring tiles, which find them in the L2 only
@@ -1344,7 +1361,8 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
         // instances: 437 us with it, 202 without).
         const bool narrow = pp.args.cmap && pp.C * pp.es < 64;
         const bool plain = (pp.variant == VAR_PLAIN || pp.variant == VAR_TWIDDLE) && !narrow;
-        if (plan->chunk_outer) {
+        bool throughout = false;
+        if (chunked) {
             pp.nt_load = plain && pp.is_first && pp.src == BUF_IN && stream_min_bytes() > 0;
             pp.nt_store = plain && pp.is_last && pp.dst == BUF_OUT && stream_min_bytes() > 0;
         } else {
@@ -1355,17 +1373,41 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
             // accesses: arrays that alone fill the cache then stream in every
             // other pass, as one streaming end gains nothing there (32 x 2^20:
             // 236 us streaming throughout, 203 at both ends, 247 at one).
-            if (plan->passes.size() > 1 && !((d->flags & RK_FFT_FUSED_ENDS) && pp.nt_load) &&
-                !(work.size() > 1 && pp.nt_load && stream_all(pp))) {
+            throughout = several && pp.nt_load &&
+                         ((d->flags & RK_FFT_FUSED_ENDS) || (work.size() > 1 && stream_all(pp)));
+            if (several && !throughout) {
                 const int ends = plain ? stream_ends(pp, work.size()) : 0;
                 pp.nt_load = (ends & 1) && pp.is_first && pp.src == BUF_IN;
                 pp.nt_store = (ends & 2) && pp.is_last && pp.dst == BUF_OUT;
             }
         }
+        // A pass from the caller's input to the output, or in place, whose
+        // rows of instances are no whole lines: without hints the parts meet
+        // in a cache (us, with / without: 32 x 1000 x 1000 over axis 1 134 /
+        // 119, 100 x 90 x 7500 405 / 268, 100 x 256 x 2001 405 / 243, 100 x
+        // 64 x 8001 217 / 210; the columns of 300 x 1000 x 1000 over axes 1
+        // and 2, in chunks, 1139 / 1029).
+        if (!throughout && (!several || pp.src == pp.dst)) {
+            pp.nt_load = pp.nt_load && whole_units(pp, tile(pp), false, 128);
+            pp.nt_store = pp.nt_store && whole_units(pp, tile(pp), true, 128);
+        }
+    }
+    // The ends of a chain along one axis stream both or, when one of them has
+    // broken units of 64 bytes, neither (us, both / stores not / neither:
+    // 100 x 750000 968 / 707 / 680, 2000 x 30000 633 / 502 / 451, 40 x 900000
+    // 369 / 345 / 321); half lines are no loss here (100 x 10^6 in chunks
+    // 774 / 888 / 824, 60 x 250000 complex128 193 / 233 / 210).
+    if (several && work.size() == 1 && !(d->flags & RK_FFT_FUSED_ENDS)) {
+        PassPlan &first = plan->passes.front(), &last = plan->passes.back();
+        if ((first.nt_load && !whole_units(first, tile(first), false, 64)) ||
+            (last.nt_store && !whole_units(last, tile(last), true, 64)))
+            first.nt_load = last.nt_store = false;
+    }
+    for (PassPlan& pp : plan->passes) {
         pp.pipe = pipe_enabled() && pp.args.load_mode == RK_MODE_DIRECT && pp.loops.empty();
         pp.half = half_enabled() && (int64_t)pp.C * lds_pitch_host(pp.L) * pp.es <= 80 * 1024;
         pp.occ = occ_min_length() >= 0 ? occ_min_length() > 0 && pp.L >= occ_min_length() : occ_default(pp);
-        rc = find_pair_kernel(pp, d->flags, plan->chunk_outer != 0);
+        rc = find_pair_kernel(pp, d->flags, chunked);
         if (rc == RK_OK && !pp.pair_C) rc = find_kernel(pp, d->flags);
         if (rc != RK_OK) return rc;
         set_xcd_group(pp);

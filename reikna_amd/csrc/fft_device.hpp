@@ -1345,6 +1345,12 @@ __device__ __forceinline__ rk_u32 instances_left(const rk_pass_args& a, rk_u64 i
     return hi ? 0x7fffffffu : (rk_u32)left;
 }
 
+// Elements of a FLAT side of a tile with `left` instances left: C*L, fewer in
+// the last tile.
+template <int L, int C> __device__ __forceinline__ rk_u32 flat_elements(rk_u32 left) {
+    return (left < (rk_u32)C ? left : (rk_u32)C) * (rk_u32)L;
+}
+
 // One tile (instances tile*C ... tile*C + C - 1) computed by threads
 // tid = 0 ... C*T - 1 with `lds` of at least tile_lds_bytes<L, C, HALF, ES>()
 // bytes (ES = sizeof the IO policy's element type).
@@ -1441,17 +1447,23 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
     } else if (load_mode == RK_MODE_FLAT) {
         // instance-linear block of C*L elements, no pre-ops
         const rk_i64 base = a.in_off + (rk_i64)inst0 * L;
-        const rk_u32 left = instances_left(a, inst0);
+        const rk_u32 left = instances_left(a, inst0), last = flat_elements<L, C>(left) - 1;
 #pragma unroll
         for (int it = 0; it < R0; ++it) {
+            // a lane past the last instance loads another element (the last, or
+            // a transformation's first); its results are never stored.  The
+            // bound on the element keeps the address a 32-bit offset from one
+            // uniform base: with a select of the tile's first element all 16
+            // held 64-bit addresses at once, the 48-point tile 145 VGPRs (now
+            // 114) and three work-groups per CU instead of four: 87381 x 48
+            // 15.1 -> 13.1 us, 37449 x 112 17.2 -> 15.1, 174762 x 24 12.7 ->
+            // 11.6.
             const int e = tid + it * NT;
             const int ce = e / L, p = e - ce * L;
-            // a lane past the last instance loads the tile's first element; its
-            // results are never stored
             const bool ok = (rk_u32)ce < left;
             if constexpr (HasPtr<IO>::value) {
-                const rk_u64 at = reinterpret_cast<rk_u64>(table<X>(a.in) + base);
-                g[it] = io.load_p(at + (ok ? (rk_u32)e * (rk_u32)sizeof(X) : 0u));
+                const rk_u32 n = (rk_u32)e < last ? (rk_u32)e : last;
+                g[it] = io.load_p(reinterpret_cast<rk_u64>(table<X>(a.in) + base) + n * (rk_u32)sizeof(X));
             } else if constexpr (IO::kBranchFree) {
                 g[it] = io.load(a, ok ? inst0 + ce : inst0, ok ? p : 0, 0, ok ? base + e : base);
             } else {
@@ -1553,13 +1565,13 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
         lds_exchange<SPLIT, QL * RL, R0>(lds, v, g, last_out, [&](int it) { return flat_lds<L, NT, LP>(tid, it); });
         adjust_all<R0>(a, g, adjust);
         const rk_i64 base = a.out_off + (rk_i64)inst0 * L;
-        const rk_u32 left = instances_left(a, inst0);
+        const rk_u32 left = instances_left(a, inst0), end = flat_elements<L, C>(left);
         auto store_all = [&](auto keep) {
 #pragma unroll
             for (int it = 0; it < R0; ++it) {
                 const int e = tid + it * NT;
                 const int ce = e / L, k = e - ce * L;
-                if (keep(ce)) {
+                if (keep(e, ce)) {
                     if constexpr (HasPtr<IO>::value)
                         io.store_p(reinterpret_cast<rk_u64>(table<X>(a.out) + base) + (rk_u32)e * (rk_u32)sizeof(X),
                                    g[it]);
@@ -1569,8 +1581,8 @@ __device__ __forceinline__ void fft_pass_tile(const rk_pass_args& a, const IO& i
             }
         };
         // one uniform branch, not one per value
-        if (left >= (rk_u32)C) store_all([](int) { return true; });
-        else store_all([&](int ce) { return (rk_u32)ce < left; });
+        if (left >= (rk_u32)C) store_all([](int, int) { return true; });
+        else store_all([&](int e, int ce) { return HasPtr<IO>::value ? (rk_u32)e < end : (rk_u32)ce < left; });
     } else {
         constexpr int NO = lower_out<V>(R0) ? R0 / 2 : R0;
         lds_exchange<SPLIT, QL * RL, NO>(lds, v, g, last_out, [&](int it) { return cs * LP + col_lds<T>(ps, it); });

@@ -105,7 +105,7 @@ def radix_list(length: int) -> list[int]:
             if f and front == seq[f - 1]:
                 continue
             t = length // front
-            if t > 1024 or (length <= 4096 and t > 256) or t < 32 <= t0 or (t < 10 and t0 >= 20):
+            if t > 1024 or (length <= 4096 and t > 256) or t < 32 <= t0 or (t < 10 and t0 >= 20) or (t < 6 and t0 >= 15):
                 continue
             if any(-(-(length // r) // t) * r > 20 for r in seq):
                 continue
@@ -155,7 +155,7 @@ def tile_c_row(length: int) -> int:
 
 def tile_c_col(length: int) -> int:
     t = threads_per_instance(length)
-    c = max(16, (tile_c_row(length) // 16) * 16)
+    c = max(32 if length <= 96 and t <= 16 else 16, (tile_c_row(length) // 16) * 16)
     while c > 1 and (c * t > 1024 or c * lds_pitch(length) * 8 > 159 * 1024):
         c //= 2
     return c

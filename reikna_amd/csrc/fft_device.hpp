@@ -426,15 +426,16 @@ __host__ __device__ constexpr long long radix_cost(int L, const int* r, int n, b
 // padded slots apart in LDS, pays for its bank conflicts.  The prime powers stay
 // unless that is 10 % cheaper, and rows of at least 32 threads keep them (below
 // 32 a contiguous side is staged through LDS), as those of at least 20 do
-// rather than go below 10 (30000 x 81: 9.7 us with 27 threads, 10.6 with 9).  Composite radices leave 1000 =
-// 10 * 10 * 10 where prime powers gave 8 * 5 * 5 * 5 and 1080 = 12 * 15 * 6
+// rather than go below 10 (30000 x 81: 9.7 us with 27 threads, 10.6 with 9) and
+// those of at least 15 rather than go below 6 (30000 x 75: 9.4 us with 15
+// threads, 12.2 with 5, whose tiles of 51 instances leave a CU four
+// work-groups).  Composite radices leave 1000 = 10 * 10 * 10 where prime powers gave 8 * 5 * 5 * 5 and 1080 = 12 * 15 * 6
 // for 8 * 5 * 3 * 3 * 3: fewer exchanges and fewer idle threads.  At most 20
 // values per thread, and at most 256 threads up to 4096 points (the batch
 // kernel's work-group).  Prime powers / composite radices, us: rows 4096 x
 // 1000 15.3 / 12.9, 2048 x 2000 22.4 / 16.0, 500 x 1200 9.4 / 6.0; columns
 // 1440 x 1440 17.5 / 11.9, 200 x 360000 543 / 509; 192 cubed 68.0 / 62.1,
-// 160 cubed 45.2 / 40.9; the one loss seen, 32 x 1000 x 1000 over axis 1,
-// 127 / 133 (8 * 5 * 5 * 5 gives 1000 threads to a tile, 10 * 10 * 10 800).
+// 160 cubed 45.2 / 40.9.
 __host__ __device__ constexpr RadixList make_radix_list(int L) {
     const int kR[12] = {16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
     RadixList best = prime_power_list(L);
@@ -464,7 +465,7 @@ __host__ __device__ constexpr RadixList make_radix_list(int L) {
         for (int f = 0; f < n; ++f) {   // each distinct radix in front
             if (f > 0 && idx[f] == idx[f - 1]) continue;
             const int T = L / kR[idx[f]];
-            if (T > 1024 || (L <= 4096 && T > 256) || (T < 32 && T0 >= 32) || (T < 10 && T0 >= 20)) continue;
+            if (T > 1024 || (L <= 4096 && T > 256) || (T < 32 && T0 >= 32) || (T < 10 && T0 >= 20) || (T < 6 && T0 >= 15)) continue;
             int r[16] = {kR[idx[f]]}, m = 1;
             for (int s = 0; s < n; ++s)
                 if (s != f) r[m++] = kR[idx[s]];

@@ -214,7 +214,12 @@ int tile_c_col(int L) {
     if (any)
         if (int f = forced_tile("RK_COL_TILE", L)) return f;
     int T = threads_per_instance(L);
-    int C = std::max(16, (default_tile_c_row(L) / 16) * 16);
+    // Complex64 instances of at most 96 points and 16 threads: tiles of at least
+    // 32 (whole pairs of lines; 16 / 32 instances, us: 63 x 800000 over axis 0
+    // 176 / 158, 70 x 800000 198 / 174, 75 x 80000 24.1 / 21.1, 90 x 200000
+    // 59.0 / 55.1; without nontemporal hints 100 x 90 x 7500 over axis 1 268 /
+    // 277, 100 x 63 x 7500 181 / 184).
+    int C = std::max(t_elem_bytes == 8 && L <= 96 && T <= 16 ? 32 : 16, (default_tile_c_row(L) / 16) * 16);
     while (C > 1 && ((int64_t)C * T > 1024 || (int64_t)C * lds_pitch_host(L) * t_elem_bytes > 159 * 1024)) C /= 2;
     // Complex128 tiles of more than 256 points stop at 256 threads (69 KB of
     // LDS, whole exchanges): 8 against 16 instances of 512 points 361 / 379 us

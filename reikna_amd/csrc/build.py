@@ -161,20 +161,20 @@ def tile_c_col(length: int) -> int:
     return c
 
 
-def pair_tile_widths(length: int) -> list[int]:
-    """Instances per tile of a pair kernel: 16 .. 64 with at most 256 threads
-    (16 always), as rk_fft_plan.cpp pair_tile picks them; none for plans of
-    more than 16 values per thread or many idle lanes."""
+PAIR_TILE = 16                       # instances per tile of a pair kernel (rk_fft_plan.cpp kPairTile)
+
+
+def has_pair_tile(length: int) -> bool:
+    """Whether rk_fft_plan.cpp pair_tile ever picks pairs of this length: at most
+    16 values per thread, few idle lanes, at most 800 threads."""
     t = threads_per_instance(length)
     if any(-(-(length // r) // t) * r > 16 for r in radix_list(length)):
-        return []
+        return False
     idle = 0
     for r in radix_list(length):
         slots = -(-(length // r) // t) * t
         idle += 1000 - 1000 * (length // r) // slots
-    if idle > 250 or 8 * t > 800:
-        return []
-    return [c for c in (16, 32, 64) if c == 16 or c // 2 * t <= 256]
+    return idle <= 250 and PAIR_TILE // 2 * t <= 800
 
 
 def catalog_lengths() -> list[int]:
@@ -270,15 +270,13 @@ def catalog_entries() -> list[tuple[int, int, int]]:
         if (length <= 1024 and c * threads_per_instance(length) == 1024 and base in (VAR_PLAIN, VAR_TWIDDLE)
                 and v & (VAR_MODE_DD | VAR_MODE_DF)):
             ents.add((length, c, v | VAR_OCC))
-    # column passes with two instances per thread (rk_fft_plan.cpp pair_tile),
-    # for every tile width the planner may pick
+    # column passes with two instances per thread (rk_fft_plan.cpp pair_tile)
     for length, c, v in list(ents):
         base = v & ~(nt | VAR_MODE_DD | VAR_MODE_DF)
         if (PAIR_MIN <= length <= FACTOR_MAX and c == tile_c_col(length)
                 and base in (VAR_PLAIN, VAR_TWIDDLE) and v & (VAR_MODE_DD | VAR_MODE_DF)
-                and (v & VAR_MODE_DD or radix_list(length)[0] % 2 == 0)):
-            for cp in pair_tile_widths(length):
-                ents.add((length, cp, v | VAR_PAIR))
+                and (v & VAR_MODE_DD or radix_list(length)[0] % 2 == 0) and has_pair_tile(length)):
+            ents.add((length, PAIR_TILE, v | VAR_PAIR))
     # plans over several axes stream their first pass's loads (contiguous rows)
     # and their last pass's stores (strided columns) when their arrays near the
     # Infinity Cache (rk_fft_plan.cpp stream_ends)
@@ -296,9 +294,8 @@ def catalog_entries() -> list[tuple[int, int, int]]:
             if length <= FACTOR_MAX:
                 if length <= 1024 and tile_c_col(length) * threads_per_instance(length) == 1024:
                     ents.add((length, tile_c_col(length), VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_OCC))
-                if PAIR_MIN <= length:
-                    for cp in pair_tile_widths(length):
-                        ents.add((length, cp, VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_PAIR))
+                if PAIR_MIN <= length and has_pair_tile(length):
+                    ents.add((length, PAIR_TILE, VAR_PLAIN | VAR_NT_STORE | VAR_MODE_DD | VAR_PAIR))
             if length & (length - 1) and threads_per_instance(length) >= 32:
                 ents.add((length, tile_c_row(length), VAR_PLAIN | VAR_NT_LOAD | VAR_MODE_DD))
             if length & (length - 1) and length >= 8 and threads_per_instance(length) < 32:

@@ -894,6 +894,15 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
     return jit_pass_kernel(pp.L, pp.C, want | mbit, &pp.jit, &pp.threads, &pp.lds_bytes);
 }
 
+// RK_PAIR=0 turns the pair kernels off.
+static bool pair_enabled() {
+    static const bool v = [] {
+        const char* e = getenv("RK_PAIR");
+        return !(e && *e && atoi(e) == 0);
+    }();
+    return v;
+}
+
 // Instances per tile of the pair kernel of a pass (two adjacent instances per
 // thread, RK_VAR_PAIR), or 0 when the pass cannot run as pairs: complex64
 // column tiles with DIRECT loads and DIRECT or FLAT stores whose innermost
@@ -915,13 +924,7 @@ static int find_kernel(PassPlan& pp, uint32_t flags) {
 // 86.8 / 93.0, 800 x 800 85.2 / 88.8, 100 x 640000 499 / 544), work-groups of
 // over 800 threads (32 x 625 x 800 56.6 / 66.3) or rows that are no whole
 // lines (32 x 1000 x 1000 134 / 133, 16 x 10^6 128 / 141).
-static bool pair_enabled() {
-    static const bool v = [] {
-        const char* e = getenv("RK_PAIR");
-        return !(e && *e && atoi(e) == 0);
-    }();
-    return v;
-}
+constexpr int kPairTile = 16;
 
 static int pair_tile(const PassPlan& pp, bool chunked) {
     const rk_pass_args& a = pp.args;
@@ -932,10 +935,10 @@ static int pair_tile(const PassPlan& pp, bool chunked) {
     if (t_tuning && t_tuning->col_tile > 0) return 0;
     if (pp.L < 512 || pp.L > 1200) return 0;
     const bool dd = mbit == VAR_MODE_DD;
-    const rk_u64 tiles16 = a.n_inst / 16;   // tiles of the pair kernel
+    const rk_u64 tiles = a.n_inst / kPairTile;
     // the other tile has parts of 128-byte lines, or a CU to itself
     const bool poor = pp.C < 16 || tile_lds_bytes_host(pp.L, pp.C, pp.es) > 80 * 1024;
-    if (!pp.nt_load && !pp.nt_store && !(dd && (poor || pp.L == 1024) && tiles16 >= 512)) return 0;
+    if (!pp.nt_load && !pp.nt_store && !(dd && (poor || pp.L == 1024) && tiles >= 512)) return 0;
     const rkfft::RadixList rl = rkfft::make_radix_list(pp.L);
     if (!dd && (pp.L % 2 || rl.r[0] % 2)) return 0;   // two positions per store
     // at most 16 values of each instance per thread, and few lanes without a
@@ -960,20 +963,15 @@ static int pair_tile(const PassPlan& pp, bool chunked) {
         if (a.in_sa != 1 || dd) return 0;
     }
     // lengths other than powers of two: tiles of whole 128-byte lines only
-    if (inner % ((pp.L & (pp.L - 1)) ? 16 : 2)) return 0;
-    // 256 threads where the tile's LDS leaves two work-groups per CU, and
-    // whole tiles per outer index (chunked chains start at tile boundaries)
+    if (inner % ((pp.L & (pp.L - 1)) ? kPairTile : 2)) return 0;
+    // 16 instances: eight pairs of T >= 32 threads, two work-groups per CU
     const int T = threads_per_instance(pp.L);
-    if (8 * T > 800 || rkfft::pair_lds_bytes(pp.L, 16, T) > 80 * 1024) return 0;
-    const rk_u64 per_outer = a.dim_I * a.dim_NS * a.dim_H;
-    int C = 64;
-    while (C > 16 && ((C / 2) * T > 256 || per_outer % (rk_u64)C || rkfft::pair_lds_bytes(pp.L, C, T) + pp.L * 8 > 80 * 1024))
-        C /= 2;
+    if (kPairTile / 2 * T > 800 || rkfft::pair_lds_bytes(pp.L, kPairTile, T) > 80 * 1024) return 0;
     // In a chunked chain the tiles must not cross outer indices: a chunk's
     // workspace is rebased, and a tile that reached past the chunk (its lanes
     // past the last instance take instance 0's addresses) would read outside
     // it.
-    return chunked && per_outer % (rk_u64)C ? 0 : C;
+    return chunked && a.dim_I * a.dim_NS * a.dim_H % kPairTile ? 0 : kPairTile;
 }
 
 // The pair kernel of a pass: the catalogue's, or one from the run-time
@@ -1358,7 +1356,7 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
     // loads, its last pass's stores): the intermediate stays in the Infinity
     // Cache between the passes of a chunk.
     const bool several = plan->passes.size() > 1, chunked = plan->chunk_outer != 0;
-    auto tile = [&](const PassPlan& pp) { return pair_tile(pp, chunked) ? pair_tile(pp, chunked) : pp.C; };
+    auto tile = [&](const PassPlan& pp) { return pair_tile(pp, chunked) ? kPairTile : pp.C; };
     for (PassPlan& pp : plan->passes) {
         // A column tile of less than 64 bytes per row leaves parts of its cache
         // lines to the neighbouring tiles, which find them in the L2 only

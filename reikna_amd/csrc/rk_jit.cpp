@@ -9,6 +9,7 @@
 #include <string>
 #include <tuple>
 
+#include "fft_device.hpp"
 #include "rk_internal.hpp"
 #include "rk_embedded.inc"
 
@@ -57,7 +58,9 @@ int jit_pass_kernel(int L, int C, int variant, hipFunction_t* fn, int* threads, 
         RK_HIP(hipModuleGetFunction(&k.fn, k.module, "rk_jit_pass"));
         k.threads = nt;
         const int es = (variant & VAR_F64) ? 16 : 8;
-        k.lds = (variant & VAR_HALF) ? tile_lds_bytes_host(L, C, es) / 2 : tile_lds_bytes_host(L, C, es);
+        k.lds = (variant & VAR_PAIR)   ? rkfft::pair_lds_bytes(L, C, T)
+                : (variant & VAR_HALF) ? tile_lds_bytes_host(L, C, es) / 2
+                                       : tile_lds_bytes_host(L, C, es);
         it = cache.emplace(key, k).first;
     }
     *fn = it->second.fn;

@@ -1222,8 +1222,6 @@ RK_HD constexpr int flat_lds(int tid, int it) {
     }
 }
 
-// Padded LDS position of element it of a thread at position ps < T of an
-// instance on a staged COLUMN / ROW side: ps + it*T.
 // The same for a pair tile, whose threads take two consecutive positions at a
 // time: value 2*it + b is position e % L + b of pair e / L, e = 2*(tid + it*NT)
 // (L even, so both positions are on one side of every padding slot).
@@ -1240,6 +1238,8 @@ RK_HD constexpr int flat_pair_lds(int tid, int it, int b) {
     }
 }
 
+// Padded LDS position of element it of a thread at position ps < T of an
+// instance on a staged COLUMN / ROW side: ps + it*T.
 template <int T> RK_HD constexpr int col_lds(int ps, int it) { return lds_pad_add<(T < 16 ? T : 16)>(ps, it * T); }
 
 // LOWER: the upper half of the first stage's inputs is zero (lower_in).

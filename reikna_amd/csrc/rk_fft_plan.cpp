@@ -1139,16 +1139,22 @@ int build_tables(TableBuilder& tb, PassPlan& pp, const AxisPass& ap, int64_t nre
     const bool needs_chirp = (ap.pre_ops & RK_PRE_CHIRP) || (ap.post_ops & RK_POST_CHIRP);
     if (needs_chirp) {
         // exp(-i pi (n^2 mod 2N) / N): the phase index is an exact integer
-        // zeros behind its end up to the middle of the axis (the kernels'
-        // upper positions are never loaded): padded inputs times these vanish
-        std::vector<cd> ch(std::max<int64_t>(nreal, ap.Nax), cd(0, 0));
+        // zeros behind its end, up to the middle of the axis: padded inputs times
+        // these vanish.  Beyond it a side reads the table only where an odd
+        // radix keeps its whole axis (lower_in / lower_out: the first stage's
+        // of a chirp input; the last's, or the first's that stages it, of an
+        // output).
+        const rkfft::RadixList rl = rkfft::make_radix_list(pp.L);
+        const bool whole = rl.r[0] % 2 || ((ap.post_ops & RK_POST_CHIRP) && rl.r[rl.n - 1] % 2);
+        const int64_t size = std::max<int64_t>(nreal, whole ? ap.Nax : ap.Nax / 2);
+        std::vector<cd> ch(size, cd(0, 0));
         const int64_t two_n = 2 * nreal;
         for (int64_t k = 0; k < nreal; ++k) {
             const unsigned __int128 sq = (unsigned __int128)k * (unsigned __int128)k;
             const int64_t ph = (int64_t)(sq % (unsigned __int128)two_n);
             ch[k] = unit_root(ph, two_n);   // exp(-2 pi i ph / 2N) = exp(-i pi ph / N)
         }
-        pp.chirp_off = add_table(tb, pp, "chirp" + std::to_string(nreal) + "_" + std::to_string(ap.Nax), ch);
+        pp.chirp_off = add_table(tb, pp, "chirp" + std::to_string(nreal) + "_" + std::to_string(size), ch);
     }
     const bool needs_bspec = ap.blue_single || (ap.post_ops & RK_POST_KMUL_CONJ);
     if (needs_bspec) {

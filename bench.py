@@ -64,13 +64,13 @@ FWD_INV = ("c1",)   # a step is the forward and the inverse transform
 # requests to the memory fabric, reads served by the Infinity Cache included.
 # Each entry names the profile summary it comes from.
 MEASURED_TRAFFIC = {
-    "c2b": (2.181e9, "profiles/fft_pass_c2b_64x2p20.md"),
+    "c2b": (2.151e9, "profiles/fft_pass_c2b_64x2p20.md"),
     "c1": (3.407e7, "profiles/fft_pass_c1_1024x1024.md"),
-    "c2a": (5.372e8, "profiles/fft_pass_c2a_256cubed.md"),
-    "c3-1000": (6.581e7, "profiles/fft_pass_c3_4096x1000.md"),
-    "c3-997": (6.629e7, "profiles/fft_pass_c3_4096x997_bluestein.md"),
+    "c2a": (8.058e8, "profiles/fft_pass_c2a_256cubed.md"),
+    "c3-1000": (6.572e7, "profiles/fft_pass_c3_4096x1000.md"),
+    "c3-997": (6.617e7, "profiles/fft_pass_c3_4096x997_bluestein.md"),
     "c3-12288": (1.612e9, "profiles/fft_pass_c3_4096x12288.md"),
-    "c4": (4.134e8, "profiles/fft_batch_c4_512_uneven.md"),
+    "c4": (4.202e8, "profiles/fft_batch_c4_512_uneven.md"),
 }
 
 

@@ -1395,10 +1395,15 @@ static int plan_create(const rk_fft_desc* d, rk_fft_plan** out) {
         // in a cache (us, with / without: 32 x 1000 x 1000 over axis 1 134 /
         // 119, 100 x 90 x 7500 405 / 268, 100 x 256 x 2001 405 / 243, 100 x
         // 64 x 8001 217 / 210; the columns of 300 x 1000 x 1000 over axes 1
-        // and 2, in chunks, 1139 / 1029).
+        // and 2, in chunks, 1139 / 1029).  Tiles of two lines and more break
+        // few of theirs: rows of whole half lines then keep the hints (1000
+        // instances of 8 points 90 / 94, of 64 97 / 104, of 128 102 / 107;
+        // narrower tiles of 160 116 / 112, of 256 111 / 107, of 512 122 / 109;
+        // 500 of 256 points in complex128 104 / 110).
         if (!throughout && (!several || pp.src == pp.dst)) {
-            pp.nt_load = pp.nt_load && whole_units(pp, tile(pp), false, 128);
-            pp.nt_store = pp.nt_store && whole_units(pp, tile(pp), true, 128);
+            const int unit = tile(pp) * pp.es >= 256 ? 64 : 128;
+            pp.nt_load = pp.nt_load && whole_units(pp, tile(pp), false, unit);
+            pp.nt_store = pp.nt_store && whole_units(pp, tile(pp), true, unit);
         }
     }
     // The ends of a chain along one axis stream both or, when one of them has

@@ -22,7 +22,11 @@ def hints(shape, axes, dtype="complex64", strides=None, out_strides=None):
     ((32, 1000, 1008), (1,), "complex64", [BOTH]),
     ((100, 256, 2001), (1,), "complex64", [NONE]),
     ((100, 256, 2000), (1,), "complex64", [BOTH]),
-    ((100, 250, 1004), (1,), "complex128", [NONE]),
+    ((524, 64, 1000), (1,), "complex64", [BOTH]),       # tiles of 512 bytes: whole half lines do
+    ((524, 64, 1001), (1,), "complex64", [NONE]),
+    ((131, 256, 1000), (1,), "complex64", [NONE]),      # tiles of 128 bytes
+    ((100, 250, 1003), (1,), "complex128", [NONE]),
+    ((100, 250, 1004), (1,), "complex128", [BOTH]),
     ((100, 250, 1000), (1,), "complex128", [BOTH]),
     ((2048, 65536), (0,), "complex64", [BOTH]),         # 64-byte tiles of whole rows
     ((300, 1000, 1000), (1, 2), "complex64", [LOAD, NONE]),       # chunked, in place
